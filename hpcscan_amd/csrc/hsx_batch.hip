@@ -172,7 +172,7 @@ static int batch_setup_shape(hsx_batch *b, const hsx_grid *grids, const void *co
     const int total = off[ns];
     const unsigned grid = (unsigned)(((int64_t)total + 7) / 8 * 8);
     b->step = [=](int parity, hipStream_t s) -> int {
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(LX, BY), K::LDS, s, (const TiledArgs<TS> *)dargs[parity],
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(LX * BY), K::LDS, s, (const TiledArgs<TS> *)dargs[parity],
                            (const int *)doff, ns);
         HSX_LAUNCHED("k_tiled_batch");
         return HSX_OK;
@@ -269,7 +269,7 @@ static int batch_setup_persistent(hsx_batch *b, const hsx_grid *grids, const voi
     const int np = (int)parts;
     const unsigned grid = (unsigned)((parts + 7) / 8 * 8);
     b->step = [=](int parity, hipStream_t st) -> int {
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(LX, BY), K::LDS, st, (const TiledArgs<TS> *)dargs[parity],
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(LX * BY), K::LDS, st, (const TiledArgs<TS> *)dargs[parity],
                            (const BatchSeg *)dseg, (const int *)dso, np);
         HSX_LAUNCHED("k_tiled_batch_seg");
         return HSX_OK;

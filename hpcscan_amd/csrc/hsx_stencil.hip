@@ -9,6 +9,7 @@
 // hsx_ac2_step / hsx_laplacian / hsx_fd_d2 use the LDS-tiled kernels of
 // hsx_stencil_tiled.hip when the grid fits them, else these.
 #include "hsx_internal.h"
+#include "hsx_route.h"
 #include "hsx_stencil_point.h"
 
 namespace hsx {
@@ -96,7 +97,7 @@ int hsx_fd_d2(const hsx_grid *g, int axis, const void *u, void *w, void *stream)
     if (rc) return rc;
     if (axis < 0 || axis >= g->dim) return fail(HSX_ERR_INVALID, "axis %d with dim %d", axis, g->dim);
     hipStream_t s = stream_of(stream);
-    if (kernel_family() != HSX_KERNEL_REF) {
+    if (kernel_family() != HSX_KERNEL_REF && tiled_pays(g)) {
         rc = tiled_fd_d2(g, axis, u, w, s);
         if (rc != HSX_ERR_UNSUPPORTED || kernel_family() == HSX_KERNEL_TILED) return rc;
     }
@@ -124,7 +125,7 @@ int hsx_fd_d1(const hsx_grid *g, int axis, const void *u, void *w, void *stream)
     if (rc) return rc;
     if (axis < 0 || axis >= g->dim) return fail(HSX_ERR_INVALID, "axis %d with dim %d", axis, g->dim);
     hipStream_t s = stream_of(stream);
-    if (kernel_family() != HSX_KERNEL_REF) {
+    if (kernel_family() != HSX_KERNEL_REF && tiled_pays(g)) {
         rc = tiled_fd_d1(g, axis, u, w, s);
         if (rc != HSX_ERR_UNSUPPORTED || kernel_family() == HSX_KERNEL_TILED) return rc;
     }
@@ -151,7 +152,7 @@ int hsx_laplacian(const hsx_grid *g, const void *u, void *w, void *stream)
     int rc = stencil_checks(g, {{u, "u"}, {w, "w"}});
     if (rc) return rc;
     hipStream_t s = stream_of(stream);
-    if (kernel_family() != HSX_KERNEL_REF) {
+    if (kernel_family() != HSX_KERNEL_REF && tiled_pays(g)) {
         rc = tiled_laplacian(g, u, w, s);
         if (rc != HSX_ERR_UNSUPPORTED || kernel_family() == HSX_KERNEL_TILED) return rc;
     }
@@ -186,7 +187,7 @@ int hsx_ac2_step_to(const hsx_grid *g, void *out, const void *prn, const void *p
     if (rc) return rc;
     if (prn == prc || out == prc) return fail(HSX_ERR_INVALID, "prn / out and prc must be different grids");
     hipStream_t s = stream_of(stream);
-    if (kernel_family() != HSX_KERNEL_REF) {
+    if (kernel_family() != HSX_KERNEL_REF && tiled_pays(g)) {
         rc = tiled_ac2_step(g, out, prn, prc, coef, s);
         if (rc != HSX_ERR_UNSUPPORTED || kernel_family() == HSX_KERNEL_TILED) return rc;
     }

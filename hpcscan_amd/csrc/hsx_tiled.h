@@ -59,8 +59,9 @@ struct TiledArgs {
     const void *coef;         // MODE_AC2 only
     int64_t n1, n2, n12;      // row length, rows per plane, plane stride
     int64_t s1, e1, s2, e2, s3, e3;
-    int64_t t1s;              // n1 origin of the first tile (multiple of VW)
+    int64_t t1s;              // n1 origin of the first tile: <= s1, and whole vectors from the row's end
     int ntx, nty, nchunk, chunk;
+    int lx;                   // lanes of a tile along n1 (<= LX): the row in ntx even parts
     int nt;                   // 1: prn / coef / output streamed with nontemporal accesses
     // MODE_AC2: the free surface folded into the step (0 = none):
     //  FOLD_PRC  prc is read as if its boundary planes were zero,
@@ -108,15 +109,27 @@ struct Tiled {
     static constexpr size_t LDS = PLANES_BYTES + RING_H + RING_C;
 };
 
+// 16 bytes of a grid as a clang vector, aligned to one element only: rows whose
+// length is not a multiple of the vector (odd sizes, odd halo widths) start
+// anywhere, and gfx950 loads and stores dwordx4 at any dword address
+template <typename TS, int VW>
+using NVec = TS __attribute__((ext_vector_type(VW), aligned(sizeof(TS))));
+
 template <typename TS, int VW>
 __device__ __forceinline__ Pack<TS, VW> vload(const TS *p)
 {
-    return *reinterpret_cast<const Pack<TS, VW> *>(p);
+    Pack<TS, VW> r;
+    __builtin_memcpy(&r, p, sizeof(r));
+    return r;
 }
 
-// the same 16 bytes as a clang vector, for the nontemporal builtins
+// (a copy, not a vector store: the compiler would merge it with the vstore_nt
+// of the other branch and drop the nontemporal hint of both)
 template <typename TS, int VW>
-using NVec = TS __attribute__((ext_vector_type(VW)));
+__device__ __forceinline__ void vstore(TS *p, const Pack<TS, VW> &x)
+{
+    __builtin_memcpy(p, &x, sizeof(x));
+}
 
 template <typename TS, int VW>
 __device__ __forceinline__ Pack<TS, VW> vload_nt(const TS *p)
@@ -168,7 +181,10 @@ __device__ __forceinline__ int xcd_logical(int total)
 }
 
 // one workgroup: planes [z0, z1) of tile 'tile' of the grid described by a
-template <typename TS, typename TC, int R, int VW, int LX, int BY, int MODE, bool RING_, bool FOLD = false>
+// (PART: the workgroup may hold more threads than the tile's a.lx x BY; the
+// rest only meet the barriers)
+template <typename TS, typename TC, int R, int VW, int LX, int BY, int MODE, bool RING_, bool FOLD = false,
+          bool PART = false>
 __device__ __forceinline__ void tiled_body_tz(const TiledArgs<TC> &a, int tile, int64_t z0, int64_t z1)
 {
     using K = Tiled<TS, TC, R, VW, LX, BY, MODE, RING_>;
@@ -181,12 +197,16 @@ __device__ __forceinline__ void tiled_body_tz(const TiledArgs<TC> &a, int tile, 
     V *ring_h = reinterpret_cast<V *>(hsx_lds_raw + K::PLANES_BYTES);
     V *ring_c = reinterpret_cast<V *>(hsx_lds_raw + K::PLANES_BYTES + K::RING_H);
 
-    const int tx = threadIdx.x, ty = threadIdx.y;
+    const int lx = a.lx;
+    const int row_ = (int)(threadIdx.x / (unsigned)lx);
+    const int tx = (int)threadIdx.x - row_ * lx;
+    const bool act = !PART || row_ < BY;
+    const int ty = act ? row_ : BY - 1;
 
-    const int64_t t1 = a.t1s + (int64_t)(tile % a.ntx) * (LX * VW);            // first n1 index of the tile
+    const int64_t t1 = a.t1s + (int64_t)(tile % a.ntx) * (lx * VW);            // first n1 index of the tile
     const int64_t i1 = t1 + tx * VW;                                           // first n1 index of this lane
     const int64_t t2s = a.s2 + (int64_t)(tile / a.ntx) * BY;                   // first n2 row of the tile
-    const int64_t i2 = t2s + ty;
+    const int64_t i2 = act ? t2s + ty : a.n2;                                  // n2: no row
 
     const bool lane_in_row = i1 + VW - 1 < a.n1;        // vector fully inside the row
     const bool row_ok = i2 < a.n2;
@@ -195,15 +215,22 @@ __device__ __forceinline__ void tiled_body_tz(const TiledArgs<TC> &a, int tile, 
 
     // Addressing: plane base (uniform, scalar registers) + 32-bit byte offset of
     // the lane inside the plane (the host checks that a plane is below 4 GiB).
+    // The bases lie one vector below the plane and the offsets one above: the
+    // first vector of a row starts below it where the row's length is not a
+    // multiple of VW (a.t1s), and the points before it are the end of the row
+    // before.  That read stays inside the grid: the tile's own rows and halo
+    // columns are on rows >= s2 >= 1, and the n2 halo rows, which reach row 0,
+    // are read on planes >= s3 >= 1 only.
     const int64_t pstride = a.n12 * ES;
-    const char *ub = reinterpret_cast<const char *>(a.u);
-    const char *pb = reinterpret_cast<const char *>(a.prn_in);
-    const char *cb = reinterpret_cast<const char *>(a.coef);
-    char *ob = reinterpret_cast<char *>(a.out);
+    constexpr int64_t BIAS = VW * ES;
+    const char *ub = reinterpret_cast<const char *>(a.u) - BIAS;
+    const char *pb = reinterpret_cast<const char *>(a.prn_in) - BIAS;
+    const char *cb = reinterpret_cast<const char *>(a.coef) - BIAS;
+    char *ob = reinterpret_cast<char *>(a.out) - BIAS;
     auto at = [&](const char *base, int64_t z, uint32_t off) -> const TS * {
         return reinterpret_cast<const TS *>((base + z * pstride) + (uint64_t)off);
     };
-    const uint32_t col = (uint32_t)((i1 + i2 * n1) * ES);
+    const uint32_t col = (uint32_t)((i1 + i2 * n1) * ES + BIAS);
 
     // ---- folded free surface (FOLD instances; the closed form of
     // Grid::applyBoundaryCondition ANTI_MIRROR, src/grid.cpp:3065-3230): an inner
@@ -212,7 +239,7 @@ __device__ __forceinline__ void tiled_body_tz(const TiledArgs<TC> &a, int tile, 
     constexpr bool FK = FOLD && mode_ac2(MODE);
     constexpr bool FMA = mode_fma(MODE);
     const int fold = FK ? a.fold : 0;
-    const int64_t tw = (int64_t)LX * VW;
+    const int64_t tw = (int64_t)lx * VW;
     auto in_range = [](int64_t x, int64_t lo, int64_t hi) { return x >= lo && x < hi; };
     // the tile (with its halo) holds a boundary column / row of a folded face (uniform)
     const bool edge_t = FK && (in_range(a.fb[0], t1 - HL, t1 + tw + HL) || in_range(a.fb[1], t1 - HL, t1 + tw + HL) ||
@@ -283,21 +310,21 @@ __device__ __forceinline__ void tiled_body_tz(const TiledArgs<TC> &a, int tile, 
         const int row = h < R ? h : BY + h;                // LDS row
         const int64_t hi2 = t2s + row - R;
         hrow_lds[k] = row;
-        hrow_off[k] = (uint32_t)((i1 + hi2 * n1) * ES);
-        hrow_ok[k] = K::NEED_Y && h < 2 * R && hi2 < a.n2 && lane_in_row;
+        hrow_off[k] = (uint32_t)((i1 + hi2 * n1) * ES + BIAS);
+        hrow_ok[k] = K::NEED_Y && act && h < 2 * R && hi2 < a.n2 && lane_in_row;
         hrow[k] = vzero<TS, VW>();
     }
     const bool left = K::NEED_X && tx < NHG;
-    const bool right = K::NEED_X && tx >= LX - NHG;
-    const int64_t hc_i1 = left ? t1 - HL + tx * VW : t1 + LX * VW + (tx - (LX - NHG)) * VW;
-    const int hc_lds = left ? tx * VW : HL + LX * VW + (tx - (LX - NHG)) * VW;
-    const bool hc_ok = (left || right) && row_ok && hc_i1 >= 0 && hc_i1 + VW - 1 < a.n1;
-    const uint32_t hc_off = (uint32_t)((hc_i1 + i2 * n1) * ES);
+    const bool right = K::NEED_X && tx >= lx - NHG;
+    const int64_t hc_i1 = left ? t1 - HL + tx * VW : t1 + lx * VW + (tx - (lx - NHG)) * VW;
+    const int hc_lds = left ? tx * VW : HL + lx * VW + (tx - (lx - NHG)) * VW;
+    const bool hc_ok = (left || right) && row_ok && hc_i1 > -VW && hc_i1 + VW - 1 < a.n1;
+    const uint32_t hc_off = (uint32_t)((hc_i1 + i2 * n1) * ES + BIAS);
 
     // ring slots owned by this thread
     // (threads that own no halo get in-range addresses too, so that the ring is
     // read without branches; what they read is not used)
-    const int rc_idx = left ? tx : right ? NHG + (tx - (LX - NHG)) : 0;
+    const int rc_idx = left ? tx : right ? NHG + (tx - (lx - NHG)) : 0;
     auto ring_h_at = [&](int slot, int k) -> V * {
         return ring_h + ((slot * 2 * R + (ty + k * BY) % (2 * R)) * LX + tx);
     };
@@ -404,7 +431,7 @@ __device__ __forceinline__ void tiled_body_tz(const TiledArgs<TC> &a, int tile, 
                 if ((f >> v) & (f >> 8) & 1) o[v] = (((f >> (4 + v)) | (f >> 9)) & 1) ? -(TS)0 : -res.v[v];
         }
         if (near2) {
-            uint32_t y = threadIdx.y;
+            uint32_t y = (uint32_t)ty;
             asm volatile("" : "+v"(y));
             const int r = (int)t2s + (int)y;
             for (int side = 0; side < 2; side++) {
@@ -419,7 +446,7 @@ __device__ __forceinline__ void tiled_body_tz(const TiledArgs<TC> &a, int tile, 
             }
         }
         if (near1) {
-            uint32_t x = threadIdx.x;
+            uint32_t x = (uint32_t)tx;
             asm volatile("" : "+v"(x));
             const int c0 = (int)t1 + (int)x * VW;
             TS *o = reinterpret_cast<TS *>((ob + z * pstride) + (uint64_t)col);
@@ -461,7 +488,7 @@ __device__ __forceinline__ void tiled_body_tz(const TiledArgs<TC> &a, int tile, 
             // ring (loaded R planes ago) or from the registers loaded last plane
             TS *pl = lds + buf * K::PLANE;
             if (K::NEED_LDS) {
-                *reinterpret_cast<V *>(pl + (ty + R) * W + HL + tx * VW) = cur;
+                if (act) *reinterpret_cast<V *>(pl + (ty + R) * W + HL + tx * VW) = cur;
                 if constexpr (RING) {
 #pragma unroll
                     for (int k = 0; k < NHR; k++) {
@@ -619,7 +646,7 @@ __device__ __forceinline__ void tiled_body_tz(const TiledArgs<TC> &a, int tile, 
                     if (a.nt)
                         vstore_nt<TS, VW>(outp, res);
                     else
-                        *reinterpret_cast<V *>(outp) = res;
+                        vstore<TS, VW>(outp, res);
                 } else {
 #pragma unroll
                     for (int v = 0; v < VW; v++)
@@ -634,9 +661,9 @@ __device__ __forceinline__ void tiled_body_tz(const TiledArgs<TC> &a, int tile, 
                     const int64_t *ib = a.img_box;
                     if (z >= ib[4] && z <= ib[5] && i2 >= ib[2] && i2 <= ib[3] && i1 + VW - 1 >= ib[0] &&
                         i1 <= ib[1]) {
-                        const V q0 = vload<TS, VW>(at(reinterpret_cast<const char *>(a.img_q[0]), z, col));
-                        const V q1 = vload<TS, VW>(at(reinterpret_cast<const char *>(a.img_q[1]), z, col));
-                        const V q2 = vload<TS, VW>(at(reinterpret_cast<const char *>(a.img_q[2]), z, col));
+                        const V q0 = vload<TS, VW>(at(reinterpret_cast<const char *>(a.img_q[0]) - BIAS, z, col));
+                        const V q1 = vload<TS, VW>(at(reinterpret_cast<const char *>(a.img_q[1]) - BIAS, z, col));
+                        const V q2 = vload<TS, VW>(at(reinterpret_cast<const char *>(a.img_q[2]) - BIAS, z, col));
                         double *gp = a.img_grad + (z * a.n12 + i2 * n1 + i1);
 #pragma unroll
                         for (int v = 0; v < VW; v++) {
@@ -653,14 +680,15 @@ __device__ __forceinline__ void tiled_body_tz(const TiledArgs<TC> &a, int tile, 
 }
 
 // one workgroup: tile / chunk number 'logical' of the grid described by a
-template <typename TS, typename TC, int R, int VW, int LX, int BY, int MODE, bool RING_, bool FOLD = false>
+template <typename TS, typename TC, int R, int VW, int LX, int BY, int MODE, bool RING_, bool FOLD = false,
+          bool PART = false>
 __device__ __forceinline__ void tiled_body(const TiledArgs<TC> &a, int logical)
 {
     const int tile = logical % (a.ntx * a.nty);
     const int chunk = logical / (a.ntx * a.nty);
     const int64_t z0 = a.s3 + (int64_t)chunk * a.chunk;
     const int64_t z1 = min(z0 + a.chunk, a.e3 + 1);    // planes [z0, z1)
-    tiled_body_tz<TS, TC, R, VW, LX, BY, MODE, RING_, FOLD>(a, tile, z0, z1);
+    tiled_body_tz<TS, TC, R, VW, LX, BY, MODE, RING_, FOLD, PART>(a, tile, z0, z1);
 }
 
 template <typename TS, typename TC, int R, int VW, int LX, int BY, int MODE, bool RING_, bool FOLD = false>
@@ -685,7 +713,7 @@ __global__ void __launch_bounds__(LX *BY) k_tiled_batch(const TiledArgs<TC> *__r
     int s = 0;
     while (s + 1 < nshots && off[s + 1] <= logical) s++;
     const TiledArgs<TC> a = grids[s];
-    tiled_body<TS, TC, R, VW, LX, BY, MODE, RING_>(a, logical - off[s]);
+    tiled_body<TS, TC, R, VW, LX, BY, MODE, RING_, false, true>(a, logical - off[s]);
 }
 
 // The batched step as one persistent launch: as many workgroups as the device
@@ -711,7 +739,7 @@ __global__ void __launch_bounds__(LX *BY) k_tiled_batch_seg(const TiledArgs<TC> 
     for (int k = so[part]; k < so[part + 1]; k++) {
         const BatchSeg sg = seg[k];
         if (k > so[part]) __syncthreads();              // the previous segment's last plane is read
-        tiled_body_tz<TS, TC, R, VW, LX, BY, MODE, RING_>(grids[sg.shot], sg.tile, sg.z0, sg.z1);
+        tiled_body_tz<TS, TC, R, VW, LX, BY, MODE, RING_, false, true>(grids[sg.shot], sg.tile, sg.z0, sg.z1);
     }
 }
 
@@ -808,6 +836,19 @@ inline int64_t chunk_one_round(int64_t N3, int R, int64_t tiles, int64_t slots)
 
 int device_cus(void);   // compute units of the current device (hsx_runtime.hip)
 
+// lanes of a tile: the row in ntx even parts (whole 128-byte lines each where
+// there are several), where that leaves out at least an eighth of LX lanes
+// that would lie past the row; a lane serves one halo column only
+template <int R, int VW, int LX>
+inline int tile_lanes(int64_t span1, int ntx)
+{
+    constexpr int NHG = (R + VW - 1) / VW;
+    int lx = (int)(((span1 + VW - 1) / VW + ntx - 1) / ntx);
+    if (ntx > 1) lx = (lx + 7) / 8 * 8;
+    lx = std::max(lx, std::max(8, 2 * NHG));
+    return 8 * lx <= 7 * LX ? lx : LX;
+}
+
 // resident workgroups per CU of a kernel instance (once per instantiation;
 // also lifts the 64 KiB default cap on dynamic LDS where the tile needs more)
 template <typename KERN>
@@ -865,7 +906,7 @@ inline int fill_tiled_args(const hsx_grid *g, void *out, const void *prn_in, con
     a.n1 = g->n1;
     a.n2 = g->n2;
     a.n12 = g->n1 * g->n2;
-    if (a.n12 * (int64_t)sizeof(TS) >= ((int64_t)1 << 32))
+    if (a.n12 * (int64_t)sizeof(TS) + 16 >= ((int64_t)1 << 32))
         return fail(HSX_ERR_UNSUPPORTED, "tiled kernels: one n3 plane must stay below 4 GiB");
     a.s1 = g->inner[0];
     a.e1 = g->inner[1];
@@ -873,9 +914,12 @@ inline int fill_tiled_args(const hsx_grid *g, void *out, const void *prn_in, con
     a.e2 = g->inner[3];
     a.s3 = g->inner[4];
     a.e3 = g->inner[5];
-    a.t1s = (a.s1 / VW) * VW;
+    // vectors counted back from the row's end, so that none reaches past it; a
+    // multiple of VW where n1 is one, else down to -(VW - 1)
+    a.t1s = a.s1 - (a.s1 + VW - a.n1 % VW) % VW;
     const int64_t span1 = a.e1 - a.t1s + 1;
     a.ntx = (int)((span1 + LX * VW - 1) / (LX * VW));
+    a.lx = tile_lanes<R, VW, LX>(span1, a.ntx);
     a.nty = (int)((a.e2 - a.s2 + 1 + BY - 1) / BY);
     const int64_t N3 = a.e3 - a.s3 + 1;
     const int64_t tiles = (int64_t)a.ntx * a.nty;
@@ -922,7 +966,7 @@ inline int launch_tiled(const hsx_grid *g, void *out, const void *prn_in, const 
     if (rc) return rc;
     const int64_t nblk = (int64_t)a.ntx * a.nty * a.nchunk;
     const unsigned grid = (unsigned)(((nblk + 7) / 8) * 8);
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(LX, BY), K::LDS, s, a);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3((unsigned)(a.lx * BY)), K::LDS, s, a);
     HSX_LAUNCHED("k_tiled");
     return HSX_OK;
 }
@@ -988,12 +1032,20 @@ inline int launch_tiled_by(const hsx_grid *g, void *out, const void *prn_in, con
     return launch_tiled<TS, TC, R, VW, LX, 8, MODE, false, FOLD>(g, out, prn_in, u, coef, s, cfg);
 }
 
-// alignment and size conditions of the tiled kernels
-inline int tiled_fits(const hsx_grid *g, int vw_elems, size_t elem)
+// size and alignment conditions of the tiled kernels.  They take rows of any
+// length and buffers at any element address (vload; hsx_route.h says which
+// grids are sent here).  Against one thread per point the fused step on 403 x
+// 307 x 255 at order 4 (rows of 407 points) went from 193 to 90 us, on 401 x
+// 403 x 399 at order 16 from 1064 to 311 us, on 601 x 603 x 599 at order 10
+// from 2683 to 923 us, FP64 301 x 299 x 303 at order 8 from 429 to 233 us.  A
+// request for the tiled family (HSX_KERNEL_TILED) and the folded free surface
+// still ask for whole vectors.
+inline int tiled_fits(const hsx_grid *g, int vw_elems, uintptr_t addr_bits, bool aligned_only)
 {
     if (g->dim != 3) return fail(HSX_ERR_UNSUPPORTED, "tiled kernels need a 3D grid");
+    if (!aligned_only) return HSX_OK;
     if (g->n1 % vw_elems) return fail(HSX_ERR_UNSUPPORTED, "n1 %% %d != 0", vw_elems);
-    (void)elem;
+    if (addr_bits % 16) return fail(HSX_ERR_UNSUPPORTED, "buffers not 16-byte aligned");
     return HSX_OK;
 }
 
@@ -1027,10 +1079,9 @@ inline int run_tiled_shape(const hsx_grid *g, void *out, const void *prn_in, con
         using TS = decltype(ts);
         using TC = decltype(tc);
         constexpr int VW = 16 / sizeof(TS);
-        int rc = tiled_fits(g, VW, sizeof(TS));
+        int rc = tiled_fits(g, VW, (uintptr_t)out | (uintptr_t)prn_in | (uintptr_t)u | (uintptr_t)coef,
+                            FOLD || kernel_family() == HSX_KERNEL_TILED);
         if (rc) return rc;
-        if (((uintptr_t)out | (uintptr_t)prn_in | (uintptr_t)u | (uintptr_t)coef) % 16)
-            return fail(HSX_ERR_UNSUPPORTED, "buffers not 16-byte aligned");
         TileCfg cfg = cfg_in;
         int lx = pick_lx(g, VW, cfg);
         // FP32 defaults measured per size (HIP events, kernel alone): the fused

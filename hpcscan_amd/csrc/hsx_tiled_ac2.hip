@@ -5,6 +5,7 @@
 #include <mutex>
 #include <vector>
 
+#include "hsx_route.h"
 #include "hsx_tiled.h"
 
 namespace hsx {
@@ -16,6 +17,12 @@ TileCfg tile_forced(void)
 {
     std::lock_guard<std::mutex> lk(g_tile_mu);
     return g_tile;
+}
+
+bool tile_shape_forced(void)
+{
+    const TileCfg c = tile_forced();
+    return c.lx || c.by || c.chunk || c.flags;
 }
 
 int set_tile(int lx, int by, int chunk, int flags)
@@ -106,6 +113,8 @@ extern "C" int hsx_autotune(const hsx_grid *g, int reps, int shape[4], float *be
     if (rc) return rc;
     if (reps < 1 || reps > 1000) return fail(HSX_ERR_INVALID, "reps %d not in 1..1000", reps);
     if (g->dim != 3) return fail(HSX_ERR_UNSUPPORTED, "the tiled kernels (and the tuner) need a 3D grid");
+    if (g->n1 % (g->storage == HSX_FP64 ? 2 : 4))
+        return fail(HSX_ERR_UNSUPPORTED, "the tuner needs rows of whole 16-byte vectors");
     if ((rc = ensure_init())) return rc;
     hipStream_t s = stream_of(nullptr);
     const size_t es = g->storage == HSX_FP64 ? 8 : 4;
