@@ -333,8 +333,13 @@ __device__ __forceinline__ void bc_zero_face(TS *u, const FaceSet &fs, int face)
 // is stored back as read. 1000^3 FP32 order 8: 0.075 ms for both n1 faces,
 // against 0.111 ms through k_bc_mirror + k_bc_zero (a second pass over the
 // same 64-byte sectors of 2 x 10^6 rows).
-template <typename TS, int NH>
-__device__ __forceinline__ void bc_n1_rows(TS *u, const Face &lo, const Face &hi, int sides, uint32_t t)
+// skip(c2, c3): rows left out (the one-launch form).
+struct NoRow {
+    __device__ bool operator()(int, int) const { return false; }
+};
+template <typename TS, int NH, typename SKIP = NoRow>
+__device__ __forceinline__ void bc_n1_rows(TS *u, const Face &lo, const Face &hi, int sides, uint32_t t,
+                                           SKIP skip = SKIP())
 {
     constexpr int VW = 16 / sizeof(TS), R = NH * VW;
     using NV = TS __attribute__((ext_vector_type(VW)));
@@ -345,6 +350,7 @@ __device__ __forceinline__ void bc_n1_rows(TS *u, const Face &lo, const Face &hi
     const uint32_t row = ns == 2 ? t >> 1 : t;
     const int side = ns == 2 ? (int)(t & 1) : ((sides & 1) ? 0 : 1);
     const uint32_t io = row / NB, ib = row - io * NB;
+    if (skip((int)f.bs + (int)ib, (int)f.os + (int)io)) return;
     NV *r = reinterpret_cast<NV *>(u + (f.os + (int64_t)io) * f.so + (f.bs + (int64_t)ib) * f.sb);
     NV w[NH + 1];
     if (side == 0) {
@@ -424,6 +430,195 @@ __global__ void __launch_bounds__(256) k_bc_n1_mirror_batch(TS *const *u, const 
     const uint32_t m = blockIdx.x - nb_n1;
     const int face = (int)(m / nb1);
     if (face < fs[s].n) bc_mirror_face(u[s], fs[s], face, m % nb1, nb1);
+}
+
+// ---- free surface, all faces in one launch ----------------------------------------
+// The closed form above needs its second launch only because the planes it
+// zeroes hold mirror sources: a point on a boundary plane of axis a is the
+// source of the halos of the axes before a (of those after a it gives -0,
+// unread).  Here the thread that zeroes such a point first writes those halos
+// itself, and the mirror threads leave them out, so that no thread reads a
+// point that another one writes: one launch in any order.  A point on planes
+// of two axes belongs to the lower one's plane.  The faces' boundary planes
+// must be the first / last inner planes (fs_one_launch).
+// Bound by launches on small grids, by the row ends of the n1 faces (a sector or
+// two each) on large ones.  Two launches before, us: 61^3 FP32 order 8 6.4 ->
+// 3.8, 200^3 7.0 -> 5.3, 403 x 307 x 255 order 4 15.2 -> 6.5, 601 x 600 x 580
+// order 10 51 -> 33, FP64 500^3 order 12 46.5 -> 43.5, 1000^3 order 8 111 -> 109,
+// 1501 x 2001 (2D) 5.6 -> 3.3.
+// Geometry: inner ranges per axis (s, e: the boundary planes), halo widths of
+// the masked faces (0: not masked), first block of each n2 / n3 face.
+struct BcOne {
+    int s[3], e[3];
+    int h[3][2];
+    int64_t n1, n12;
+    uint32_t first[5];       // first block of faces n2 low, n2 high, n3 low, n3 high, and the end
+    int sides;               // n1 faces by bc_n1_rows (bit 0 / 1), 0: by points
+};
+
+template <typename TS>
+struct VecOf {
+    static constexpr int W = 16 / sizeof(TS);
+    using U = TS __attribute__((ext_vector_type(W), aligned(sizeof(TS))));       // any element address
+};
+
+// c lies on a masked boundary plane of the axis
+__device__ __forceinline__ bool on_plane(const BcOne &b, int axis, int c)
+{
+    return (b.h[axis][0] && c == b.s[axis]) || (b.h[axis][1] && c == b.e[axis]);
+}
+
+// -v, or -0 on the masked n1 boundary planes / the whole row
+template <typename TS, typename V>
+__device__ __forceinline__ V mirror_of(const BcOne &b, const V &v, int i1, bool zrow)
+{
+    V w;
+#pragma unroll
+    for (int e = 0; e < VecOf<TS>::W; e++) w[e] = zrow || on_plane(b, 0, i1 + e) ? -(TS)0.0 : -v[e];
+    return w;
+}
+
+// store the elements of w that lie in the inner n1 range
+template <typename TS, typename V>
+__device__ __forceinline__ void store_in(const BcOne &b, TS *p, const V &w, int i1)
+{
+    constexpr int VW = VecOf<TS>::W;
+    if (i1 >= b.s[0] && i1 + VW - 1 <= b.e[0]) {
+        *reinterpret_cast<typename VecOf<TS>::U *>(p) = w;
+    } else {
+#pragma unroll
+        for (int e = 0; e < VW; e++)
+            if (i1 + e >= b.s[0] && i1 + e <= b.e[0]) p[e] = w[e];
+    }
+}
+
+// One n2 (A = 1) or n3 (A = 2) face in 16-byte groups along n1, item t: its
+// boundary plane (k = 0) and its halo rows (k = 1 .. h).  The last group of a
+// row may take in a few points past the inner range; they are read (inside the
+// grid: these rows are inner rows) and not written.
+template <typename TS, int A>
+__device__ __forceinline__ void bc1_face(TS *u, const BcOne &b, int side, uint32_t t)
+{
+    constexpr int VW = VecOf<TS>::W, O = 3 - A;           // O: the outer axis
+    using U = typename VecOf<TS>::U;
+    const int64_t so = A == 1 ? b.n12 : b.n1, sa = A == 1 ? b.n1 : b.n12;
+    const int h = b.h[A][side], plane = side == 0 ? b.s[A] : b.e[A], g0 = b.s[0] / VW;
+    const uint32_t NG = (uint32_t)(b.e[0] / VW - g0 + 1), H = (uint32_t)(h + 1);
+    const uint32_t r = t / NG, io = r / H;
+    const int k = (int)(r - io * H), i1 = (g0 + (int)(t - r * NG)) * VW, o = b.s[O] + (int)io;
+    if (o > b.e[O]) return;
+    // n2 faces: the halo rows on an n3 plane belong to that plane's threads; n3
+    // faces: the plane's rows on an n2 plane to the n2 plane's threads
+    const bool oz = on_plane(b, O, o);
+    if (oz && (A == 1) == (k > 0)) return;
+    const int d = side == 0 ? k : -k;
+    TS *p = u + (o * so + (plane + d) * sa + i1);         // the mirror source, or the plane's own points
+    const U v = *reinterpret_cast<const U *>(p);
+    if (k > 0) {
+        store_in<TS, U>(b, p - 2 * d * sa, mirror_of<TS, U>(b, v, i1, A == 2 && oz), i1);
+        return;
+    }
+    if (A == 2) {
+        // the n2 halos that mirror this row
+        const int d0 = o - b.s[1], d1 = b.e[1] - o;
+        if (d0 >= 1 && d0 <= b.h[1][0]) store_in<TS, U>(b, p - 2 * d0 * b.n1, mirror_of<TS, U>(b, v, i1, false), i1);
+        if (d1 >= 1 && d1 <= b.h[1][1]) store_in<TS, U>(b, p + 2 * d1 * b.n1, mirror_of<TS, U>(b, v, i1, false), i1);
+    }
+    // the n1 halos that mirror points of this group
+    if (i1 <= b.s[0] + b.h[0][0] || i1 + VW - 1 >= b.e[0] - b.h[0][1]) {
+#pragma unroll
+        for (int e = 0; e < VW; e++) {
+            const int d0 = i1 + e - b.s[0], d1 = b.e[0] - (i1 + e);
+            if (d0 >= 1 && d1 >= 0 && d0 <= b.h[0][0]) p[e - 2 * d0] = -v[e];
+            if (d1 >= 1 && d0 >= 0 && d1 <= b.h[0][1]) p[e + 2 * d1] = -v[e];
+        }
+    }
+    U z;
+#pragma unroll
+    for (int e = 0; e < VW; e++) z[e] = (TS)0.0;
+    store_in<TS, U>(b, p, z, i1);
+}
+
+// The n1 faces, one point per thread (R not a multiple of the vector, rows at
+// any address), item t: the boundary point (k = 0) and the halo points of a row
+template <typename TS>
+__device__ __forceinline__ void bc1_n1_points(TS *u, const BcOne &b, uint32_t t)
+{
+    const int h0 = b.h[0][0], h1 = b.h[0][1];
+    const uint32_t H = (uint32_t)((h0 ? h0 + 1 : 0) + (h1 ? h1 + 1 : 0)), N2 = (uint32_t)(b.e[1] - b.s[1] + 1);
+    const uint32_t r = t / H, i3 = r / N2;
+    int k = (int)(t - r * H);
+    const int c2 = b.s[1] + (int)(r - i3 * N2), c3 = b.s[2] + (int)i3;
+    if (c3 > b.e[2] || on_plane(b, 1, c2) || on_plane(b, 2, c3)) return;       // the planes' threads
+    const bool lo = h0 && k <= h0;
+    if (!lo && h0) k -= h0 + 1;
+    TS *p = u + (c3 * b.n12 + c2 * b.n1 + (lo ? b.s[0] + k : b.e[0] - k));
+    if (k == 0)
+        *p = (TS)0.0;
+    else
+        p[lo ? -2 * k : 2 * k] = -*p;
+}
+
+// NH > 0: the n1 faces by 16-byte row ends (bc_n1_rows), else by points
+template <typename TS, int NH>
+__global__ void __launch_bounds__(256) k_bc_one(TS *u, BcOne b, Face lo, Face hi)
+{
+    const uint32_t bx = blockIdx.x;
+    if (bx < b.first[0]) {
+        const uint32_t t = bx * 256u + threadIdx.x;
+        if constexpr (NH > 0)
+            bc_n1_rows<TS, NH>(u, lo, hi, b.sides, t, [&](int c2, int c3) { return on_plane(b, 1, c2) || on_plane(b, 2, c3); });
+        else
+            bc1_n1_points(u, b, t);
+    } else if (bx < b.first[2]) {
+        const int side = bx >= b.first[1];
+        bc1_face<TS, 1>(u, b, side, (bx - b.first[side]) * 256u + threadIdx.x);
+    } else {
+        const int side = bx >= b.first[3];
+        bc1_face<TS, 2>(u, b, side, (bx - b.first[2 + side]) * 256u + threadIdx.x);
+    }
+}
+
+// arguments of k_bc_one; false where it does not serve the faces (a boundary
+// plane that is not the first / last inner plane, index spaces past 32 bits)
+static bool fill_bc_one(const hsx_grid *g, const FaceSet &fs, int sides, BcOne *b)
+{
+    if (g->n1 >= INT32_MAX || g->n2 >= INT32_MAX || g->n3 >= INT32_MAX) return false;
+    const int VW = g->storage == HSX_FP64 ? 2 : 4;
+    b->n1 = g->n1;
+    b->n12 = g->n1 * g->n2;
+    b->sides = sides;
+    int64_t n[3];
+    for (int a = 0; a < 3; a++) {
+        b->s[a] = (int)g->inner[2 * a];
+        b->e[a] = (int)g->inner[2 * a + 1];
+        b->h[a][0] = b->h[a][1] = 0;
+        n[a] = b->e[a] - b->s[a] + 1;
+    }
+    for (int k = 0; k < fs.n; k++) {
+        const Face &f = fs.f[k];
+        const int side = f.inner > f.he ? 0 : 1;
+        if (f.inner != g->inner[2 * f.axis + side] || f.he < f.hs) return false;
+        b->h[f.axis][side] = (int)(f.he - f.hs + 1);
+    }
+    int64_t at = 0;
+    const int64_t most = ((int64_t)1 << 31) - 256;
+    auto take = [&](int64_t items) {
+        at += (items + 255) / 256;
+        return items < most && at < most;
+    };
+    const int64_t rows = n[1] * n[2];
+    const int64_t per_row = sides ? (sides & 1) + (sides >> 1)
+                                  : (b->h[0][0] ? b->h[0][0] + 1 : 0) + (b->h[0][1] ? b->h[0][1] + 1 : 0);
+    if (!take(rows * per_row)) return false;
+    const int64_t ng = b->e[0] / VW - b->s[0] / VW + 1;
+    for (int f = 0; f < 4; f++) {
+        const int a = 1 + f / 2, h = b->h[a][f % 2];
+        b->first[f] = (uint32_t)at;
+        if (!take(h ? ng * (h + 1) * n[3 - a] : 0)) return false;
+    }
+    b->first[4] = (uint32_t)at;
+    return at > 0;
 }
 
 int n1_groups_ok(const hsx_grid *g, const void *u, const FaceSet &fs)
@@ -980,6 +1175,25 @@ int hsx_free_surface(const hsx_grid *g, void *u, int face_mask, void *stream)
     if (fs.n == 0) return HSX_OK;
     return dispatch_types(g, [&](auto ts, auto) -> int {
         using TS = decltype(ts);
+        BcOne one;
+        Face flo{}, fhi{};
+        const int n1s = closed_form ? n1_vector_sides(g, u, fs, &flo, &fhi) : 0;
+        if (closed_form && fill_bc_one(g, fs, n1s, &one)) {
+            auto go = [&](auto nh) {
+                constexpr int NH = decltype(nh)::value;
+                hipLaunchKernelGGL((k_bc_one<TS, NH>), dim3(one.first[4]), dim3(256), 0, s, (TS *)u, one, flo, fhi);
+            };
+            const Face &f = (n1s & 1) ? flo : fhi;
+            switch (n1s ? (int)((f.he - f.hs + 1) / (16 / (int64_t)sizeof(TS))) : 0) {
+            case 0: go(IC<0>()); break;
+            case 1: go(IC<1>()); break;
+            case 2: go(IC<2>()); break;
+            case 3: go(IC<3>()); break;
+            default: go(IC<4>()); break;
+            }
+            HSX_LAUNCHED("k_bc_one");
+            return HSX_OK;
+        }
         if (closed_form) {
             const unsigned nb1 = (unsigned)std::min<int64_t>((most + 255) / 256, 4096);
             const unsigned nb2 = (unsigned)std::min<int64_t>((most_plane + 255) / 256, 4096);
