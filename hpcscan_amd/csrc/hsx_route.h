@@ -6,20 +6,20 @@
 
 namespace hsx {
 
-// Rows that are not whole 16-byte vectors (odd sizes, odd halo widths): the
-// tiled kernels take them, one thread per point does as well on small grids,
-// where a launch lasts as long as one workgroup's chunk of planes.  FP32 order
-// 8, step / Laplacian / D2 along n3, one thread per point against tiled (us):
-// 101^3 8.6 / 7.1 / 4.9 against 22.1 / 17.1 / 10.6; 151^3 24.6 / 18.6 / 15.4
-// against 38.4 / 17.7 / 15.9; 201 x 203 x 199 48.6 / 39.2 / 27.7 against 41.7 /
-// 23.3 / 16.1; 301 x 299 x 303 197 / 138 / 141 against 115 / 64 / 38.
-constexpr int64_t UNALIGNED_TILED_POINTS = 6000000;
+// Grids of up to 5 MB an array run one thread per point: a launch of the tiled
+// kernels lasts as long as a workgroup's chunk of planes takes one after the
+// other, one thread per point has no such chain.  Step, Laplacian and D2 along
+// n3, one thread per point against tiled (us): FP32 order 8 61^3 3.8 / 3.7 / 3.9
+// against 17 / 15 / 9, 80^3 5.5 (step) against 5.8, 100^3 8.0 / 6.9 / 5.1 against
+// 7.4 / 7.0 / 5.7, 128^3 13.0 / 11.2 / 10.1 against 8.4 / - / -; FP64 100^3 (10
+// MB) 15.7 (step) against 9.5.
+constexpr int64_t TILED_LEAST_BYTES = 5200000;
 bool tile_shape_forced(void);   // hsx_set_tile asks for a shape (hsx_tiled_ac2.hip)
 inline bool tiled_pays(const hsx_grid *g)
 {
-    if (kernel_family() == HSX_KERNEL_TILED || tile_shape_forced()) return true;
-    if (g->n1 % (g->storage == HSX_FP64 ? 2 : 4) == 0) return true;
-    return g->n1 * g->n2 * g->n3 >= UNALIGNED_TILED_POINTS;
+    // (the contracted arithmetic exists in the tiled kernels only)
+    if (kernel_family() == HSX_KERNEL_TILED || contract_mode() || tile_shape_forced()) return true;
+    return g->n1 * g->n2 * g->n3 * (g->storage == HSX_FP64 ? 8 : 4) >= TILED_LEAST_BYTES;
 }
 
 } // namespace hsx

@@ -777,13 +777,16 @@ struct ImgReq {
 };
 extern thread_local ImgReq t_img;     // defined in hsx_tiled_ac2_img.hip
 constexpr int TILE_LDS_MAX = 163840;  // gfx950: 160 KiB of LDS per workgroup
+// internal flag of a shape: chunks that give one round of two workgroups per CU,
+// down to 4 planes (grids that lie in the caches, default_shape)
+constexpr int TILE_FILL = 256;
 
-// 64 lanes unless the tiles of 64 lanes span more than 5/4 of the n1 width
-// that tiles of 32 lanes span (their last tile mostly idle): 328^3 FP32 order
-// 8 ran 0.125 ms with 32 x 16 tiles against 0.150 ms with 64 x 16 (512 lanes'
-// width for 320 points); 608^3 and 808^3 stay faster with 64 lanes (0.75 /
-// 1.81 ms against 0.93 / 2.22 ms) although a fifth of their lanes idle
-inline int pick_lx(const hsx_grid *g, int vw, const TileCfg &cfg)
+// lanes of the widest tile: 64, or 16 / 32 where they hold the row.  The
+// Laplacian on large grids takes 32 where tiles of 64 span more than 5/4 of the
+// width of tiles of 32 (320^3 order 8 61.6 against 68 us); the widths are fitted
+// to the row afterwards (tile_lanes), and the other kernels do as well or
+// better with the wider tiles (D2 of 320^3 42-44 us against 47-51).
+inline int pick_lx(const hsx_grid *g, int vw, const TileCfg &cfg, bool narrow = false)
 {
     if (cfg.lx) return cfg.lx;
     const int64_t N1 = g->inner[1] - g->inner[0] + 1;
@@ -791,7 +794,7 @@ inline int pick_lx(const hsx_grid *g, int vw, const TileCfg &cfg)
     if (N1 <= 32 * vw) return 32;
     const int64_t w64 = (N1 + 64 * vw - 1) / (64 * vw) * (64 * vw);
     const int64_t w32 = (N1 + 32 * vw - 1) / (32 * vw) * (32 * vw);
-    return 4 * w64 > 5 * w32 ? 32 : 64;
+    return narrow && 4 * w64 > 5 * w32 ? 32 : 64;
 }
 
 // 8-row tiles: chunks of ~48 planes (at least 4R), at least 2048 workgroups
@@ -815,9 +818,9 @@ inline int64_t chunk_short(int64_t N3, int R, int64_t tiles)
 // 252 tiles on 256 slots, 3.13 ms against 3.25 ms with 64-plane chunks); 700^3
 // (132 tiles) gets 78-plane chunks, 1188 workgroups in five rounds: 1.22 ms,
 // against 1.62 ms for two chunks per tile (264 workgroups: a second round of 8)
-inline int64_t chunk_one_round(int64_t N3, int R, int64_t tiles, int64_t slots)
+inline int64_t chunk_one_round(int64_t N3, int R, int64_t tiles, int64_t slots, int64_t least = 0)
 {
-    const int64_t minc = 4 * R < N3 ? 4 * R : N3;
+    const int64_t want = least > 0 ? least : 4 * R, minc = want < N3 ? want : N3;
     int64_t best_c = N3, best_t = INT64_MAX;
     for (int64_t k = 1; k <= N3; k++) {
         const int64_t c = (N3 + k - 1) / k;
@@ -924,8 +927,10 @@ inline int fill_tiled_args(const hsx_grid *g, void *out, const void *prn_in, con
     const int64_t N3 = a.e3 - a.s3 + 1;
     const int64_t tiles = (int64_t)a.ntx * a.nty;
     constexpr bool STREAM = !Tiled<TS, TC, R, VW, LX, BY, MODE, RING>::NEED_LDS;
-    const int64_t cs = STREAM && cfg.chunk <= 0 && chunk <= 0 ? chunk_stream(N3, R, tiles, LX * BY) : 0;
+    const int64_t cs = STREAM && cfg.chunk <= 0 && chunk <= 0 && !(cfg.flags & TILE_FILL) ? chunk_stream(N3, R, tiles, LX * BY) : 0;
     const int64_t len = cfg.chunk > 0 ? std::min<int64_t>(cfg.chunk, N3)
+                        : (cfg.flags & TILE_FILL)
+                            ? chunk_one_round(N3, R, tiles, std::min<int64_t>(slots, 2 * device_cus()), 4)
                         : chunk > 0           ? std::min<int64_t>(std::max<int64_t>(chunk, 4 * R), N3)
                         : cs > 0              ? cs
                         : (BY == 16 || RING) ? chunk_one_round(N3, R, tiles, slots)
@@ -1038,8 +1043,8 @@ inline int launch_tiled_by(const hsx_grid *g, void *out, const void *prn_in, con
 // 307 x 255 at order 4 (rows of 407 points) went from 193 to 90 us, on 401 x
 // 403 x 399 at order 16 from 1064 to 311 us, on 601 x 603 x 599 at order 10
 // from 2683 to 923 us, FP64 301 x 299 x 303 at order 8 from 429 to 233 us.  A
-// request for the tiled family (HSX_KERNEL_TILED) and the folded free surface
-// still ask for whole vectors.
+// request for the tiled family (HSX_KERNEL_TILED), the folded free surface and
+// the contracted arithmetic (whose results differ) still ask for whole vectors.
 inline int tiled_fits(const hsx_grid *g, int vw_elems, uintptr_t addr_bits, bool aligned_only)
 {
     if (g->dim != 3) return fail(HSX_ERR_UNSUPPORTED, "tiled kernels need a 3D grid");
@@ -1057,17 +1062,84 @@ bool tuned_shape(const hsx_grid *g, int mode, TileCfg *out);
 // choice (hsx_tiled_ac2.hip, which holds their instances)
 bool wide_tiles_fit(const hsx_grid *g);
 
-// The fused step's own choice of 128 x 8 tiles (with the ring) over 64 x 16:
-// where both span the same width and either one 512-point tile covers the row
-// or the row fills at least 93 % of the 128-lane tiles. Order 8 FP32, median
-// of 48 launches each on one device (128 x 8 / 64 x 16): 400^3 0.958, 460^3
-// 0.894, 500^3 0.911, 512^3 0.967, 960^3 0.992, 1000^3 0.966, 1020^3 0.988;
-// not taken at 600^3 1.202, 800^3 1.032, 900^3 1.016, 1100^3 1.053.
+// The order-4 Laplacian takes 128 x 8 tiles (with the ring) over 64 x 16 where
+// both span the same width and either one 512-point tile covers the row or the
+// row fills at least 93 % of the 128-lane tiles (1000^3 1.54 / 1.61 ms, 500^3
+// 0.189 / 0.196, 400^3 0.119 / 0.122; 700^3, not taken, 0.671 / 0.587).
 inline bool wide_by_default(const hsx_grid *g)
 {
     const int64_t N1 = g->inner[1] - g->inner[0] + 1;
     const int64_t w64 = (N1 + 255) / 256 * 256, w128 = (N1 + 511) / 512 * 512;
     return w64 == w128 && (w128 == 512 || 100 * N1 >= 93 * w128);
+}
+
+// The library's own shape (fields left 0: the general choice of run_tiled_shape
+// and fill_tiled_args).  All figures: kernel alone, us, 'was' = 16-row tiles
+// with the ring in chunks of at least 4R planes, or 64 x 8 for FP64 values.
+//
+// Grids whose arrays lie in the 256 MB Infinity Cache together (up to 200 MB)
+// are bound by the planes a workgroup streams one after the other and by CUs
+// without work, not by bytes: 8-row tiles without the ring (several workgroups
+// per CU), chunks of 4 planes or more that give one round of two workgroups per
+// CU, cached streams (the step; the kernels that write a second grid and never
+// read it again keep nontemporal ones).  Step, FP32 order 8: 128^3 8.4 (was
+// 21), 160^3 16 (27), 200^3 28.5 (39), order 16 37 (56); FP64 150^3 25 (31);
+// FP32 storage with FP64 compute 200^3 31 (41); Laplacian 160^3 12.4 (21), 256^3
+// order 12 46 (61); D2 of 160^3 8.2-8.5 (12-13).  32 lanes from order 10 on and
+// for FP64 values, which keep twice the registers (200^3 order 12 34 against 37).
+//
+// Larger grids, the fused step:
+//  * FP32 to order 8: 128 x 8 with the ring, fitted to the row, where the row is
+//    wider than one tile of 64 lanes: 300^3 84 (64 x 16: 84), 400^3 190 (195),
+//    600^3 733 (769), 700^3 1064 (1206), 800^3 1763 (1828), 1000^3 2990 (3120);
+//  * FP32 orders 14 and 16: 32 x 16 without the ring: 450 x 350 x 300 184 / 187
+//    (was 268 / 198);
+//  * FP64 up to 900 MB: 32 x 16 without the ring: 300^3 order 8 164 (177), 320 x
+//    300 x 310 order 4 / 12 166 / 184 (182 / 217); 400^3 and more 64 x 8 with it;
+//  * FP32 storage with FP64 compute: from order 10 32 x 8 without the ring,
+//    nontemporal (400^3 order 12 303, was 406); below, up to 450 MB the same in
+//    12-plane chunks (300^3 100, was 112), up to 2.4 GB 64 x 8 with the ring
+//    (400^3 order 4 / 8 217 / 228, was 234 / 267).
+template <typename TS, typename TC, int R, int MODE>
+inline TileCfg default_shape(const hsx_grid *g)
+{
+    constexpr bool FP32 = sizeof(TS) == 4 && sizeof(TC) == 4, FP64 = sizeof(TS) == 8;
+    constexpr int VW = 16 / sizeof(TS), GRIDS = mode_ac2(MODE) ? 3 : 2;
+    const int64_t bytes = g->n1 * g->n2 * g->n3 * (int64_t)sizeof(TS) * GRIDS;
+    const int64_t N1 = g->inner[1] - g->inner[0] + 1;
+    TileCfg c = {0, 0, 0, 0};
+    if (bytes <= 200000000) {
+        c.lx = std::min(pick_lx(g, VW, c), FP32 && R <= 4 ? 64 : 32);
+        c.by = 8;
+        c.flags = HSX_TILE_NO_RING | (mode_ac2(MODE) ? HSX_TILE_CACHED : HSX_TILE_NT) | TILE_FILL;
+        return c;
+    }
+    if (!mode_ac2(MODE)) return c;
+    if (FP32) {
+        if (MODE == MODE_AC2 && N1 > 64 * VW && wide_tiles_fit(g)) {
+            c.lx = 128;
+            c.by = 8;
+        } else if (R >= 7) {
+            c.lx = 32;
+            c.by = 16;
+            c.flags = HSX_TILE_NO_RING | HSX_TILE_NT;
+        }
+    } else if (FP64) {
+        if (bytes <= 900000000) {
+            c.lx = 32;
+            c.by = 16;
+            c.flags = HSX_TILE_NO_RING | HSX_TILE_NT;
+        }
+    } else if (R >= 5 || bytes <= 450000000) {
+        c.lx = 32;
+        c.by = 8;
+        c.chunk = R >= 5 ? 0 : 12;
+        c.flags = HSX_TILE_NO_RING | HSX_TILE_NT;
+    } else if (bytes <= 2400000000) {
+        c.lx = 64;
+        c.by = 8;
+    }
+    return c;
 }
 
 template <int MODE, bool FOLD = false>
@@ -1080,48 +1152,39 @@ inline int run_tiled_shape(const hsx_grid *g, void *out, const void *prn_in, con
         using TC = decltype(tc);
         constexpr int VW = 16 / sizeof(TS);
         int rc = tiled_fits(g, VW, (uintptr_t)out | (uintptr_t)prn_in | (uintptr_t)u | (uintptr_t)coef,
-                            FOLD || kernel_family() == HSX_KERNEL_TILED);
+                            FOLD || mode_fma(MODE) || kernel_family() == HSX_KERNEL_TILED);
         if (rc) return rc;
-        TileCfg cfg = cfg_in;
-        int lx = pick_lx(g, VW, cfg);
-        // FP32 defaults measured per size (HIP events, kernel alone): the fused
-        // step and the order-4 Laplacian take 128 x 8 tiles where
-        // wide_by_default holds (Laplacian order 4: 1000^3 1.54 / 1.61 ms,
-        // 500^3 0.189 / 0.196, 400^3 0.119 / 0.122; 700^3, not taken, 0.671 /
-        // 0.587); the order-8 Laplacian drops the halo ring, whose halo rows
-        // still meet in L2 with two streams instead of four (1000^3 1.84 /
-        // 1.88 ms, 800^3 1.11 / 1.24, 700^3 0.70 / 0.79, 500^3 0.237 / 0.258,
-        // 400^3 0.131 / 0.141)
-        constexpr bool fp32_vals = sizeof(TS) == 4 && sizeof(TC) == 4;
-        const bool dflt = cfg.lx == 0 && cfg.by == 0;
-        if (fp32_vals && dflt && wide_by_default(g) &&
-            (MODE == MODE_AC2 ? wide_tiles_fit(g) : MODE == MODE_LAP && R == 2))
-            lx = 128;
-        if (fp32_vals && dflt && cfg.flags == 0 && MODE == MODE_LAP && R == 4) cfg.flags = HSX_TILE_NO_RING;
-        // FP64 Laplacian: order 12 on 32 x 16 tiles (1000^3 4.54 / 4.71 ms,
-        // 800^3 2.45 / 2.71, 700^3 1.65 / 1.93, 500^3 0.535 / 0.622, 400^3
-        // 0.363 / 0.425 against 64 x 8), order 16 on 16 x 8 (1000^3 5.55 /
-        // 6.49 ms, 800^3 3.04 / 3.47, 700^3 2.08 / 2.36, 500^3 0.802 / 0.864,
-        // 400^3 0.426 / 0.486 against 32 x 16)
-        if (sizeof(TS) == 8 && dflt && MODE == MODE_LAP && lx == 64) {
-            if (R == 6) {
-                lx = 32;
-                cfg.by = 16;
-            } else if (R == 8) {
-                lx = 16;
-            }
-        }
         return dispatch_R(R, [&](auto rc_) -> int {
             constexpr int RR = decltype(rc_)::value;
+            TileCfg cfg = cfg_in;
+            const bool none = cfg.lx == 0 && cfg.by == 0 && cfg.chunk == 0 && cfg.flags == 0;
+            if (!FOLD && none) cfg = default_shape<TS, TC, RR, MODE>(g);
+            int lx = pick_lx(g, VW, cfg, MODE == MODE_LAP);
+            // the order-8 Laplacian drops the halo ring, whose halo rows still meet
+            // in L2 with two streams instead of four (1000^3 1.84 / 1.88 ms, 800^3
+            // 1.11 / 1.24, 700^3 0.70 / 0.79, 500^3 0.237 / 0.258, 400^3 0.131 / 0.141)
+            constexpr bool fp32_vals = sizeof(TS) == 4 && sizeof(TC) == 4;
+            const bool dflt = cfg.lx == 0 && cfg.by == 0;
+            if (fp32_vals && dflt && MODE == MODE_LAP && RR == 2 && wide_by_default(g)) lx = 128;
+            if (fp32_vals && dflt && cfg.flags == 0 && MODE == MODE_LAP && RR == 4) cfg.flags = HSX_TILE_NO_RING;
+            // FP64 Laplacian: order 12 on 32 x 16 tiles (1000^3 4.54 / 4.71 ms,
+            // 800^3 2.45 / 2.71, 700^3 1.65 / 1.93, 500^3 0.535 / 0.622, 400^3
+            // 0.363 / 0.425 against 64 x 8), order 16 on 16 x 8 (1000^3 5.55 /
+            // 6.49 ms, 800^3 3.04 / 3.47, 700^3 2.08 / 2.36, 500^3 0.802 / 0.864,
+            // 400^3 0.426 / 0.486 against 32 x 16)
+            if (sizeof(TS) == 8 && dflt && MODE == MODE_LAP && lx == 64) {
+                if (RR == 6) {
+                    lx = 32;
+                    cfg.by = 16;
+                } else if (RR == 8) {
+                    lx = 16;
+                }
+            }
             if (lx == 128) {
                 // 128 lanes x 8 rows with the halo ring (rows of 2 KiB, two
                 // waves each): the exact FP32 fused step and Laplacian up to
                 // order 8, where the ring's LDS fits and spills stay within
-                // TILED_SPILL_OK; the fused step's default where
-                // wide_by_default holds, otherwise on request (hsx_set_tile,
-                // the autotuner). 1000^3 order 8: 3.04-3.08 ms against
-                // 3.12-3.19 ms for 64 x 16; 500^3 0.363 against 0.394 ms;
-                // 700^3 and 800^3 6 % and 2 % slower.
+                // TILED_SPILL_OK
                 using K = Tiled<TS, TC, RR, VW, 128, 8, MODE, true>;
                 if constexpr (sizeof(TS) == 4 && sizeof(TC) == 4 && !FOLD && (MODE == MODE_AC2 || MODE == MODE_LAP) &&
                               K::RING && K::LDS <= TILE_LDS_MAX) {

@@ -61,3 +61,31 @@ def test_rows_of_any_length_bit_exact(oracle, capi, order, prec, n, lanes, rows,
         _same(dp.download(dtype), ref)
     finally:
         capi.set_tile(0, 0)
+
+
+# one grid of each class of the library's own shapes (5 MB an array, 200 MB for
+# the step's three, above by precision and order), no shape asked for
+CLASSES = [(8, "f32", (90, 85, 80)), (8, "f32", (160, 150, 141)), (12, "f32", (161, 120, 130)),
+           (8, "f64", (130, 100, 90)), (8, "f32c64", (150, 141, 100)), (8, "f32", (300, 280, 270)),
+           (4, "f32", (301, 280, 270)), (16, "f32", (300, 260, 240)), (8, "f64", (260, 240, 200)),
+           (12, "f32c64", (300, 250, 240)), (8, "f32c64", (300, 260, 250)), (4, "f32c64", (400, 330, 300))]
+
+
+@pytest.mark.parametrize("order,prec,n", CLASSES)
+def test_own_shapes_bit_exact(oracle, capi, order, prec, n):
+    dtype, c64 = PRECS[prec]
+    p, o = _layouts(oracle, 3, n, order, dtype)
+    rng = np.random.default_rng(order + n[0])
+    g = capi.hsx_grid(p, compute_fp64=c64)
+    u, coef, prn = (rng.random(p.npoint, dtype=dtype) for _ in range(3))
+    iv = oracle.inv2(p.d, dtype, compute64=c64)
+    du, dc, dp = (capi.DeviceArray.from_numpy(x) for x in (u, coef, prn))
+    ref = prn.copy()
+    oracle.pressure_fd(o, ref, u, coef, iv, compute64=c64)
+    capi.ac2_step(g, dp, du, dc)
+    _same(dp.download(dtype), ref)
+    ref = prn.copy()
+    oracle.laplacian(o, u, ref, iv, compute64=c64)
+    dp.upload(prn)
+    capi.laplacian(g, du, dp)
+    _same(dp.download(dtype), ref)
