@@ -89,13 +89,19 @@ __global__ void __launch_bounds__(256) k_srcrec(TS *u, int64_t npoint, int64_t n
 }
 
 // The source term of reverse step k (the imaging condition's -F part:
-// grad[src_i] += scale * mu^k[src_i] * f_i, for the sources inside the imaging
+// grad[src_i] -= scale * mu^k[src_i] * f_i, for the sources inside the imaging
 // box b only) and the residual of step k-1 into
 // mu^{k+1} (v[rec_i] += -1 * res_i * crec_i, in double, as k_inject) in one
 // launch: blocks [0, nb_src) take the sources, the rest the receivers; the two
 // parts touch different buffers.
+// side (imaging in pairs of steps, first of the pair: hold, then not): the pair's
+// sum over the whole grid lacks the first step's source term between its two
+// terms, so the points with a source are summed here in the order of single
+// steps, through side[i], and overwrite the pair's.
 template <typename TS>
-__global__ void __launch_bounds__(256) k_imgsrc_residual(double *grad, const TS *mu, int64_t nsrc, const int64_t *sidx,
+__global__ void __launch_bounds__(256) k_imgsrc_residual(double *grad, const TS *mu, const TS *q0, const TS *q1,
+                                                         const TS *q2, double *side, int hold, int64_t nsrc,
+                                                         const int64_t *sidx,
                                                          const TS *f, double scale, Box b, int64_t n1, int64_t n12,
                                                          uint32_t nb_src, TS *v, int64_t npoint, int64_t nrec,
                                                          const int64_t *ridx, const TS *res, const TS *crec)
@@ -106,7 +112,13 @@ __global__ void __launch_bounds__(256) k_imgsrc_residual(double *grad, const TS 
         const int64_t j = sidx[i];
         const int64_t i3 = j / n12, i2 = (j - i3 * n12) / n1, i1 = j - i3 * n12 - i2 * n1;
         if (i1 < b.s1 || i1 > b.e1 || i2 < b.s2 || i2 > b.e2 || i3 < b.s3 || i3 > b.e3) return;
-        grad[j] += scale * (double)mu[j] * (double)f[i];
+        double x = side && !hold ? side[i] : grad[j];
+        if (side) {
+            const double d2 = ((double)q0[j] - 2.0 * (double)q1[j]) + (double)q2[j];
+            x += scale * (double)mu[j] * d2;
+        }
+        x += -scale * (double)mu[j] * (double)f[i];
+        (hold ? side + i : grad + j)[0] = x;
         return;
     }
     for (int64_t i = (int64_t)(blockIdx.x - nb_src) * blockDim.x + threadIdx.x; i < nrec;
@@ -118,6 +130,34 @@ __global__ void __launch_bounds__(256) k_imgsrc_residual(double *grad, const TS 
         *p = (TS)((double)*p + x);
     }
 }
+
+// the imaging condition of two reverse steps in one pass over the gradient, for
+// the grids that the tiled kernels do not take: mu1, mu2 the two outputs in
+// order, q[0] .. q[3] the four wavefields, later ones first
+template <typename TS>
+struct Four {
+    const TS *q[4];
+};
+template <typename TS>
+__global__ void __launch_bounds__(256) k_imaging_pair(double *grad, const TS *mu1, const TS *mu2, Four<TS> w, Box b,
+                                                      int64_t n1, int64_t n12, double scale)
+{
+    const int64_t N1 = b.n1(), N2 = b.n2(), rows = N2 * b.n3();
+    for (int64_t row = (int64_t)blockIdx.x * 4 + threadIdx.y; row < rows; row += (int64_t)gridDim.x * 4) {
+        const int64_t base = (b.s2 + row % N2) * n1 + (b.s3 + row / N2) * n12 + b.s1;
+        for (int64_t k = threadIdx.x; k < N1; k += 64) {
+            const int64_t i = base + k;
+            const double a = (double)w.q[0][i], c = (double)w.q[1][i], d = (double)w.q[2][i], e = (double)w.q[3][i];
+            double x = grad[i];
+            x += scale * (double)mu1[i] * ((a - 2.0 * c) + d);
+            x += scale * (double)mu2[i] * ((c - 2.0 * d) + e);
+            grad[i] = x;
+        }
+    }
+}
+
+// sources up to which the imaging condition goes in pairs of steps
+constexpr int64_t PAIR_SRC_MAX = 4096;
 
 struct Dev {
     void *p = nullptr;
@@ -150,6 +190,21 @@ static int shot_checks(const hsx_grid *g, const void *coef, const hsx_shot *sh)
 static int zero(const hsx_grid *g, void *u, hipStream_t s)
 {
     return hsx_array_op(g, HSX_ARRAY_FILL, u, nullptr, nullptr, 0.0, s);
+}
+
+static int imaging_pair(const hsx_grid *g, double *grad, const void *mu1, const void *mu2, const void *q0,
+                        const void *q1, const void *q2, const void *q3, const Box &b, double scale, hipStream_t s)
+{
+    const int64_t rows = b.n2() * b.n3();
+    const unsigned nb = (unsigned)std::max<int64_t>(1, std::min<int64_t>((rows + 3) / 4, 1 << 20));
+    return dispatch_types(g, [&](auto ts, auto) -> int {
+        using TS = decltype(ts);
+        const Four<TS> w = {{(const TS *)q0, (const TS *)q1, (const TS *)q2, (const TS *)q3}};
+        hipLaunchKernelGGL(k_imaging_pair<TS>, dim3(nb), dim3(64, 4), 0, s, grad, (const TS *)mu1, (const TS *)mu2, w, b,
+                           g->n1, g->n1 * g->n2, scale);
+        HSX_LAUNCHED("k_imaging_pair");
+        return HSX_OK;
+    });
 }
 
 // one forward step: prev <- B(cur) step, source, record
@@ -189,7 +244,7 @@ struct hsx_adjoint_plan {
     hsx_adjoint_opts opt;
     size_t es = 4, bytes = 0, snap = 0;
     int64_t nseg = 0;
-    hsx::Dev traces, res, crec, partial, msum, m1, m2, ck, fa, fb;
+    hsx::Dev traces, res, crec, partial, msum, side, m1, m2, ck, fa, fb;
     std::vector<hsx::Dev> q;   // wavefields q^{m}, m from the segment start - 1
 };
 
@@ -234,7 +289,7 @@ static int plan_run(hsx_adjoint_plan *P, const hsx_grid *g, const void *coef, co
     const int K = P->opt.ckpt_every;
     const int fmt = P->opt.ckpt_format;
     const bool given_residual = (P->opt.flags & HSX_ADJ_RESIDUAL) != 0;
-    const size_t es = P->es, bytes = P->bytes, snap = P->snap;
+    const size_t es = P->es, snap = P->snap;
     const int64_t npoint = g->n1 * g->n2 * g->n3;
     const int64_t nt = sh->nt, nrec = sh->nrec, ntr = nt * nrec, nseg = P->nseg;
 
@@ -248,43 +303,40 @@ static int plan_run(hsx_adjoint_plan *P, const hsx_grid *g, const void *coef, co
     const double img_scale = -1.0 / (sh->dt * sh->dt);
     auto &q = P->q;
 
+    // Where the forward pass leaves q^m, m = -1 .. nt.  With full storage and
+    // storage-type checkpoints the last segment (without checkpoints the only
+    // one) goes straight to the buffers its reverse steps read, and the steps
+    // themselves write the checkpoints: neither is computed twice or copied.
+    // 16-bit checkpoints are restored in every segment, whose wavefields all
+    // carry the same rounding.
+    // (160 x 150 x 170 FP64 order 8, 60 steps: checkpoints every 10 steps 12.8 ->
+    // 7.1 ms, full storage 9.4 -> 5.7, with the imaging below and the tile shapes)
+    const bool in_place = K > 0 && fmt == HSX_CKPT_FP32;
+    const int64_t n_last = K == 0 ? 0 : in_place ? (nseg - 1) * K : nt + 2;
+    auto ck_at = [&](int64_t seg, int which) -> void * { return P->ck.c() + ((size_t)seg * 2 + which) * snap; };
+    auto loc = [&](int64_t m) -> void * {
+        if (m >= n_last - 1) return q[m - n_last + 1].p;
+        if (in_place && m % K == 0) return ck_at(m / K, 0);
+        if (in_place && (m + 1) % K == 0) return ck_at((m + 1) / K, 1);
+        return m & 1 ? P->fa.p : P->fb.p;
+    };
     auto save = [&](int64_t seg, const void *cur, const void *prev) -> int {
-        char *dst = P->ck.c() + (size_t)seg * 2 * snap;
-        if (fmt == HSX_CKPT_FP32) {
-            HSX_HIP(hipMemcpyAsync(dst, cur, bytes, hipMemcpyDeviceToDevice, s));
-            HSX_HIP(hipMemcpyAsync(dst + snap, prev, bytes, hipMemcpyDeviceToDevice, s));
-            return HSX_OK;
-        }
-        int r = hsx_ckpt_encode((const float *)cur, nullptr, npoint, dst, fmt, s);
-        if (!r) r = hsx_ckpt_encode((const float *)cur, (const float *)prev, npoint, dst + snap, fmt, s);
+        int r = hsx_ckpt_encode((const float *)cur, nullptr, npoint, ck_at(seg, 0), fmt, s);
+        if (!r) r = hsx_ckpt_encode((const float *)cur, (const float *)prev, npoint, ck_at(seg, 1), fmt, s);
         return r;
     };
     auto restore = [&](int64_t seg, void *cur, void *prev) -> int {
-        const char *src = P->ck.c() + (size_t)seg * 2 * snap;
-        if (fmt == HSX_CKPT_FP32) {
-            HSX_HIP(hipMemcpyAsync(cur, src, bytes, hipMemcpyDeviceToDevice, s));
-            HSX_HIP(hipMemcpyAsync(prev, src + snap, bytes, hipMemcpyDeviceToDevice, s));
-            return HSX_OK;
-        }
-        int r = hsx_ckpt_decode(src, npoint, fmt, nullptr, (float *)cur, s);
-        if (!r) r = hsx_ckpt_decode(src + snap, npoint, fmt, (const float *)cur, (float *)prev, s);
+        int r = hsx_ckpt_decode(ck_at(seg, 0), npoint, fmt, nullptr, (float *)cur, s);
+        if (!r) r = hsx_ckpt_decode(ck_at(seg, 1), npoint, fmt, (const float *)cur, (float *)prev, s);
         return r;
     };
 
     // ---- forward pass (traces only when the residual is formed here)
     void *tr = given_residual ? nullptr : P->traces.p;
-    if (K == 0) {
-        if ((rc = zero(g, q[0].p, s)) || (rc = zero(g, q[1].p, s))) return rc;
-        for (int64_t n = 0; n < nt; n++)
-            if ((rc = fwd_step(g, coef, sh, q[n + 2].p, q[n].p, q[n + 1].p, n, tr, es, s))) return rc;
-    } else {
-        if ((rc = zero(g, P->fa.p, s)) || (rc = zero(g, P->fb.p, s))) return rc;
-        void *prev = P->fa.p, *cur = P->fb.p;
-        for (int64_t n = 0; n < nt; n++) {
-            if (n % K == 0 && (rc = save(n / K, cur, prev))) return rc;
-            if ((rc = fwd_step(g, coef, sh, prev, prev, cur, n, tr, es, s))) return rc;
-            std::swap(prev, cur);
-        }
+    if ((rc = zero(g, loc(-1), s)) || (rc = zero(g, loc(0), s))) return rc;
+    for (int64_t n = 0; n < nt; n++) {
+        if (K > 0 && !in_place && n % K == 0 && (rc = save(n / K, loc(n), loc(n - 1)))) return rc;
+        if ((rc = fwd_step(g, coef, sh, loc(n + 1), loc(n - 1), loc(n), n, tr, es, s))) return rc;
     }
 
     // ---- residual and misfit
@@ -314,17 +366,28 @@ static int plan_run(hsx_adjoint_plan *P, const hsx_grid *g, const void *coef, co
     if (nrec > 0 &&
         (rc = hsx_inject(g, mu2, nrec, sh->rec_idx, res_at(nt), P->crec.p, -1.0, HSX_INJECT_ADD, s)))
         return rc;
-    auto back_step = [&](int64_t k, const void *qk, const void *qk1, const void *qk2) -> int {
+    // The imaging condition of two steps goes into the gradient together, in the
+    // kernel of the second one (whose input is the first one's output): the
+    // gradient, 16 bytes of traffic a point, moves half as often and two of six
+    // wavefields less are read.  200^3 FP32 order 8, 100 steps, 16-bit checkpoints
+    // every 20: 16.7 -> 14.1 ms, the imaging step 69 us every second time (a
+    // plain step 28.7).  hold: the first of a pair, imaged with the next step;
+    // q_up: its latest wavefield, in the second one.
+    const bool pairs = sh->nsrc <= PAIR_SRC_MAX;
+    auto back_step = [&](int64_t k, bool hold, const void *q_up, const void *qk, const void *qk1,
+                         const void *qk2) -> int {
         // mu^k = 2 mu^{k+1} - (mu^{k+2} - c e^k) + c L mu^{k+1}: the residual
         // went into mu^{k+2} (mu2) before the step, so that the step's output is
         // mu^k complete and the imaging condition can be taken from it
         int r = hsx_free_surface(g, mu1, 0x3F, s);
         if (!r) {
-            r = fuse_img ? tiled_ac2_step_img(g, mu2, mu1, coef, grad, qk, qk1, qk2, rim, img_scale, s)
-                         : HSX_ERR_UNSUPPORTED;
+            r = fuse_img && !hold ? tiled_ac2_step_img(g, mu2, mu1, coef, grad, qk, qk1, qk2, q_up, rim, img_scale, s)
+                                  : HSX_ERR_UNSUPPORTED;
             if (r == HSX_ERR_UNSUPPORTED) {
                 r = hsx_ac2_step(g, mu2, mu1, coef, s);                   // mu2 <- mu^k
-                if (!r) r = hsx_imaging(g, grad, mu2, qk, qk1, qk2, rim, img_scale, -1, 0.0, s);
+                if (!r && !hold)
+                    r = q_up ? imaging_pair(g, grad, mu1, mu2, q_up, qk, qk1, qk2, rimb, img_scale, s)
+                             : hsx_imaging(g, grad, mu2, qk, qk1, qk2, rim, img_scale, -1, 0.0, s);
             }
         }
         // the source term of step k (reads mu^k in mu2) and the residual of
@@ -336,10 +399,11 @@ static int plan_run(hsx_adjoint_plan *P, const hsx_grid *g, const void *coef, co
                 const uint32_t nbs = (uint32_t)((ns + 255) / 256);
                 const uint32_t nbr = (uint32_t)std::min<int64_t>((nr + 255) / 256, 1024);
                 hipLaunchKernelGGL(k_imgsrc_residual<TS>, dim3(nbs + nbr), dim3(256), 0, s, grad, (const TS *)mu2,
-                                   ns, sh->src_idx,
+                                   (const TS *)qk, (const TS *)qk1, (const TS *)qk2,
+                                   hold || q_up ? (double *)P->side.p : (double *)nullptr, (int)hold, ns, sh->src_idx,
                                    ns > 0 ? (const TS *)((const char *)sh->wavelet + (size_t)(k - 1) * ns * es)
                                           : (const TS *)nullptr,
-                                   -img_scale, rimb, g->n1, g->n1 * g->n2, nbs, (TS *)mu1, npoint, nr, sh->rec_idx,
+                                   img_scale, rimb, g->n1, g->n1 * g->n2, nbs, (TS *)mu1, npoint, nr, sh->rec_idx,
                                    nr > 0 ? (const TS *)res_at(k - 1) : (const TS *)nullptr, (const TS *)P->crec.p);
                 HSX_LAUNCHED("k_imgsrc_residual");
                 return HSX_OK;
@@ -348,20 +412,31 @@ static int plan_run(hsx_adjoint_plan *P, const hsx_grid *g, const void *coef, co
         std::swap(mu1, mu2);
         return r;
     };
-    if (K == 0) {
-        for (int64_t k = nt; k >= 1; k--)
-            if ((rc = back_step(k, q[k + 1].p, q[k].p, q[k - 1].p))) return rc;
-    } else {
-        for (int64_t seg = nseg - 1; seg >= 0; seg--) {
-            const int64_t n0 = seg * K, n1 = std::min<int64_t>(n0 + K, nt);
-            // q[j] holds q^{n0 - 1 + j}
-            if ((rc = restore(seg, q[1].p, q[0].p))) return rc;
-            for (int64_t n = n0; n < n1; n++)
-                if ((rc = fwd_step(g, coef, sh, q[n - n0 + 2].p, q[n - n0].p, q[n - n0 + 1].p, n, nullptr, es, s)))
-                    return rc;
-            for (int64_t k = n1; k > n0; k--)
-                if ((rc = back_step(k, q[k - n0 + 1].p, q[k - n0].p, q[k - n0 - 1].p))) return rc;
+    // reverse steps hi .. lo + 1 with q^m at at(m): pairs, after a single one if
+    // their number is odd
+    auto reverse = [&](int64_t hi, int64_t lo, auto at) -> int {
+        for (int64_t k = hi; k > lo; k--) {
+            const bool second = (k - lo) % 2 == 1;
+            const int r = back_step(k, pairs && !second, pairs && second && k < hi ? at(k + 1) : nullptr, at(k),
+                                    at(k - 1), at(k - 2));
+            if (r) return r;
         }
+        return HSX_OK;
+    };
+    if ((rc = reverse(nt, n_last, loc))) return rc;
+    for (int64_t seg = in_place ? nseg - 2 : nseg - 1; seg >= 0; seg--) {
+        const int64_t n0 = seg * K, n1 = std::min<int64_t>(n0 + K, nt);
+        // q^m of this segment; of the storage-type checkpoints the segment's own
+        // and the next one's serve as they lie, which leaves K - 2 steps to redo
+        auto at = [&](int64_t m) -> void * {
+            if (in_place && m <= n0) return ck_at(seg, m == n0 ? 0 : 1);
+            if (in_place && m >= n1 - 1) return loc(m);
+            return q[m - n0 + 1].p;
+        };
+        if (!in_place && (rc = restore(seg, at(n0), at(n0 - 1)))) return rc;
+        for (int64_t n = n0; n < (in_place ? n1 - 2 : n1); n++)
+            if ((rc = fwd_step(g, coef, sh, at(n + 1), at(n - 1), at(n), n, nullptr, es, s))) return rc;
+        if ((rc = reverse(n1, n0, at))) return rc;
     }
     double m = 0.0;
     HSX_HIP(hipMemcpyAsync(&m, P->msum.p, sizeof(double), hipMemcpyDeviceToHost, s));
@@ -412,23 +487,27 @@ int hsx_adjoint_plan_create(const hsx_grid *g, int64_t nt, int64_t nrec, const h
     P->es = g->storage == HSX_FP64 ? 8 : 4;
     const int64_t npoint = g->n1 * g->n2 * g->n3;
     P->bytes = (size_t)npoint * P->es;
-    const int K = opt->ckpt_every;
+    // storage-type checkpoints of every step are full storage (the same values)
+    if (opt->ckpt_every == 1 && opt->ckpt_format == HSX_CKPT_FP32) P->opt.ckpt_every = 0;
+    const int64_t K = P->opt.ckpt_every;
     const int64_t ntr = nt * nrec;
     P->nseg = K == 0 ? 0 : (nt + K - 1) / K;
-    P->snap = opt->ckpt_format == HSX_CKPT_FP32 ? P->bytes : hsx_ckpt_bytes(npoint);
+    P->snap = opt->ckpt_format == HSX_CKPT_FP32 ? (P->bytes + 255) / 256 * 256 : hsx_ckpt_bytes(npoint);
     auto bail = [&](int code) {
         delete P;
         return code;
     };
     if ((rc = P->traces.alloc(ntr * P->es)) || (rc = P->res.alloc(ntr * P->es)) || (rc = P->crec.alloc(nrec * P->es)) ||
         (rc = P->partial.alloc(4096 * sizeof(double))) || (rc = P->msum.alloc(sizeof(double))) ||
+        (rc = P->side.alloc(PAIR_SRC_MAX * sizeof(double))) ||
         (rc = P->m1.alloc(P->bytes)) || (rc = P->m2.alloc(P->bytes)))
         return bail(rc);
-    P->q.resize(K == 0 ? nt + 2 : K + 2);
+    P->q.resize((K == 0 ? nt : std::min(K, nt)) + 2);
     for (auto &x : P->q)
         if ((rc = x.alloc(P->bytes))) return bail(rc);
-    if (K > 0 && ((rc = P->ck.alloc((size_t)P->nseg * 2 * P->snap)) || (rc = P->fa.alloc(P->bytes)) ||
-                  (rc = P->fb.alloc(P->bytes))))
+    const int64_t ncks = opt->ckpt_format == HSX_CKPT_FP32 ? P->nseg - 1 : P->nseg;     // the last one: plan_run
+    if (ncks > 0 && ((rc = P->ck.alloc((size_t)ncks * 2 * P->snap)) || (rc = P->fa.alloc(P->bytes)) ||
+                     (rc = P->fb.alloc(P->bytes))))
         return bail(rc);
     *out = P;
     return HSX_OK;

@@ -170,10 +170,11 @@ int tiled_ac2_step_fma(const hsx_grid *g, void *out, const void *prn, const void
                        hipStream_t s);
 int tiled_laplacian_fma(const hsx_grid *g, const void *u, void *w, hipStream_t s);
 // the fused step in place on prn with grad += scale * new prn * (q0 - 2 q1 + q2)
-// over box (inside the inner points), in double (the adjoint's imaging condition)
+// over box (inside the inner points), in double (the adjoint's imaging condition);
+// q3 not NULL: grad += scale * prc * (q3 - 2 q0 + q1), the step before's, first
 int tiled_ac2_step_img(const hsx_grid *g, void *prn, const void *prc, const void *coef, double *grad,
-                       const void *q0, const void *q1, const void *q2, const int64_t box[6], double scale,
-                       hipStream_t s);
+                       const void *q0, const void *q1, const void *q2, const void *q3, const int64_t box[6],
+                       double scale, hipStream_t s);
 int tiled_fd_d2_x(const hsx_grid *g, const void *u, void *w, hipStream_t s);
 int tiled_fd_d2_y(const hsx_grid *g, const void *u, void *w, hipStream_t s);
 int tiled_fd_d2_z(const hsx_grid *g, const void *u, void *w, hipStream_t s);

@@ -35,7 +35,8 @@ enum TiledMode {
     // fused multiply-adds (opt-in, hsx_set_contract): not the reference's bits
     MODE_AC2_FMA = 8, MODE_LAP_FMA = 9,
     // the fused step with the adjoint's imaging condition accumulated from its
-    // output (hsx_gradient): grad += scale * out * (q0 - 2 q1 + q2) in double
+    // output (hsx_gradient): grad += scale * out * (q0 - 2 q1 + q2) in double,
+    // optionally after the same of the step before (u and its wavefields)
     MODE_AC2_IMG = 10
 };
 constexpr bool mode_ac2(int m) { return m == MODE_AC2 || m == MODE_AC2_FMA || m == MODE_AC2_IMG; }
@@ -69,8 +70,9 @@ struct TiledArgs {
     //  FOLD_HALO the output's halos of the folded faces are written (-mirror).
     int fold;
     int fb[6];                // boundary plane of each folded face (axis-major, low side first), -1 if not folded
-    // MODE_AC2_IMG: grad[i] += img_scale * out[i] * ((q0[i] - 2 q1[i]) + q2[i]) over img_box
-    const void *img_q[3];
+    // MODE_AC2_IMG: grad[i] += img_scale * out[i] * ((q0[i] - 2 q1[i]) + q2[i]) over img_box,
+    // before it (img_q[3] not NULL) grad[i] += img_scale * u[i] * ((q3[i] - 2 q0[i]) + q1[i])
+    const void *img_q[4];
     double *img_grad;
     double img_scale;
     int64_t img_box[6];
@@ -528,6 +530,26 @@ __device__ __forceinline__ void tiled_body_tz(const TiledArgs<TC> &a, int tile, 
             // order 8 1.85 ms against 1.97 ms without, order 16 1.68 / 1.85)
             __syncthreads();
 
+            // MODE_AC2_IMG: the wavefields and the gradient of these points, loaded
+            // here so that they arrive while the step is computed (the vector may
+            // hold points outside the box; it lies inside the grid like the rest)
+            V iq[4];
+            Pack<double, VW> ig;
+            bool in_img = false;
+            if constexpr (MODE == MODE_AC2_IMG) {
+                const int64_t *ib = a.img_box;
+                in_img = any_inner && z >= ib[4] && z <= ib[5] && i2 >= ib[2] && i2 <= ib[3] && i1 + VW - 1 >= ib[0] &&
+                         i1 <= ib[1];
+                if (in_img) {
+#pragma unroll
+                    for (int k = 0; k < 3; k++)
+                        iq[k] = vload<TS, VW>(at(reinterpret_cast<const char *>(a.img_q[k]) - BIAS, z, col));
+                    if (a.img_q[3])
+                        iq[3] = vload<TS, VW>(at(reinterpret_cast<const char *>(a.img_q[3]) - BIAS, z, col));
+                    ig = vload<double, VW>(a.img_grad + (z * a.n12 + i2 * n1 + i1));
+                }
+            }
+
             if (any_inner) {
                 // n1 neighbours: the row segment [tx*VW, tx*VW + VW + 2 HL) of the LDS row
                 TS xr[2 * HL + VW];
@@ -658,18 +680,25 @@ __device__ __forceinline__ void tiled_body_tz(const TiledArgs<TC> &a, int tile, 
                 if constexpr (MODE == MODE_AC2_IMG) {
                     // the imaging condition from the values just computed, in
                     // the order of k_imaging (the box lies inside the inner points)
-                    const int64_t *ib = a.img_box;
-                    if (z >= ib[4] && z <= ib[5] && i2 >= ib[2] && i2 <= ib[3] && i1 + VW - 1 >= ib[0] &&
-                        i1 <= ib[1]) {
-                        const V q0 = vload<TS, VW>(at(reinterpret_cast<const char *>(a.img_q[0]) - BIAS, z, col));
-                        const V q1 = vload<TS, VW>(at(reinterpret_cast<const char *>(a.img_q[1]) - BIAS, z, col));
-                        const V q2 = vload<TS, VW>(at(reinterpret_cast<const char *>(a.img_q[2]) - BIAS, z, col));
+                    if (in_img) {
+                        const int64_t *ib = a.img_box;
                         double *gp = a.img_grad + (z * a.n12 + i2 * n1 + i1);
 #pragma unroll
                         for (int v = 0; v < VW; v++) {
-                            if (i1 + v < ib[0] || i1 + v > ib[1]) continue;
-                            const double d2 = ((double)q0.v[v] - 2.0 * (double)q1.v[v]) + (double)q2.v[v];
-                            gp[v] += a.img_scale * (double)res.v[v] * d2;
+                            double x = ig.v[v];
+                            if (a.img_q[3]) {
+                                const double d2 = ((double)iq[3].v[v] - 2.0 * (double)iq[0].v[v]) + (double)iq[1].v[v];
+                                x += a.img_scale * (double)cur.v[v] * d2;
+                            }
+                            const double d2 = ((double)iq[0].v[v] - 2.0 * (double)iq[1].v[v]) + (double)iq[2].v[v];
+                            ig.v[v] = x + a.img_scale * (double)res.v[v] * d2;
+                        }
+                        if (i1 >= ib[0] && i1 + VW - 1 <= ib[1]) {
+                            vstore<double, VW>(gp, ig);
+                        } else {
+#pragma unroll
+                            for (int v = 0; v < VW; v++)
+                                if (i1 + v >= ib[0] && i1 + v <= ib[1]) gp[v] = ig.v[v];
                         }
                     }
                 }
@@ -770,7 +799,7 @@ extern thread_local FoldReq t_fold;   // defined in hsx_tiled_ac2.hip
 
 // imaging condition fused into the next MODE_AC2_IMG launch of this thread
 struct ImgReq {
-    const void *q[3];
+    const void *q[4];
     double *grad;
     double scale;
     int64_t box[6];
@@ -942,12 +971,12 @@ inline int fill_tiled_args(const hsx_grid *g, void *out, const void *prn_in, con
     a.fold = MODE == MODE_AC2 ? t_fold.flags : 0;   // the folded free surface: exact step only
     for (int k = 0; k < 6; k++) a.fb[k] = a.fold ? (int)t_fold.fb[k] : -1;
     if constexpr (MODE == MODE_AC2_IMG) {
-        for (int k = 0; k < 3; k++) a.img_q[k] = t_img.q[k];
+        for (int k = 0; k < 4; k++) a.img_q[k] = t_img.q[k];
         a.img_grad = t_img.grad;
         a.img_scale = t_img.scale;
         for (int k = 0; k < 6; k++) a.img_box[k] = t_img.box[k];
     } else {
-        for (int k = 0; k < 3; k++) a.img_q[k] = nullptr;
+        for (int k = 0; k < 4; k++) a.img_q[k] = nullptr;
         a.img_grad = nullptr;
         a.img_scale = 0.0;
         for (int k = 0; k < 6; k++) a.img_box[k] = 0;
