@@ -20,6 +20,7 @@
 
 #include "hsx_internal.h"
 #include "hsx_route.h"
+#include "hsx_step_end.h"
 
 namespace hsx {
 
@@ -88,47 +89,11 @@ __global__ void __launch_bounds__(256) k_srcrec(TS *u, int64_t npoint, int64_t n
     }
 }
 
-// The source term of reverse step k (the imaging condition's -F part:
-// grad[src_i] -= scale * mu^k[src_i] * f_i, for the sources inside the imaging
-// box b only) and the residual of step k-1 into
-// mu^{k+1} (v[rec_i] += -1 * res_i * crec_i, in double, as k_inject) in one
-// launch: blocks [0, nb_src) take the sources, the rest the receivers; the two
-// parts touch different buffers.
-// side (imaging in pairs of steps, first of the pair: hold, then not): the pair's
-// sum over the whole grid lacks the first step's source term between its two
-// terms, so the points with a source are summed here in the order of single
-// steps, through side[i], and overwrite the pair's.
+// the end of a reverse step alone (hsx_step_end.h)
 template <typename TS>
-__global__ void __launch_bounds__(256) k_imgsrc_residual(double *grad, const TS *mu, const TS *q0, const TS *q1,
-                                                         const TS *q2, double *side, int hold, int64_t nsrc,
-                                                         const int64_t *sidx,
-                                                         const TS *f, double scale, Box b, int64_t n1, int64_t n12,
-                                                         uint32_t nb_src, TS *v, int64_t npoint, int64_t nrec,
-                                                         const int64_t *ridx, const TS *res, const TS *crec)
+__global__ void __launch_bounds__(256) k_reverse_end(ReverseEnd<TS> r)
 {
-    if (blockIdx.x < nb_src) {
-        const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-        if (i >= nsrc) return;
-        const int64_t j = sidx[i];
-        const int64_t i3 = j / n12, i2 = (j - i3 * n12) / n1, i1 = j - i3 * n12 - i2 * n1;
-        if (i1 < b.s1 || i1 > b.e1 || i2 < b.s2 || i2 > b.e2 || i3 < b.s3 || i3 > b.e3) return;
-        double x = side && !hold ? side[i] : grad[j];
-        if (side) {
-            const double d2 = ((double)q0[j] - 2.0 * (double)q1[j]) + (double)q2[j];
-            x += scale * (double)mu[j] * d2;
-        }
-        x += -scale * (double)mu[j] * (double)f[i];
-        (hold ? side + i : grad + j)[0] = x;
-        return;
-    }
-    for (int64_t i = (int64_t)(blockIdx.x - nb_src) * blockDim.x + threadIdx.x; i < nrec;
-         i += (int64_t)(gridDim.x - nb_src) * blockDim.x) {
-        if ((uint64_t)ridx[i] >= (uint64_t)npoint) continue;
-        double x = -1.0 * (double)res[i];
-        x *= (double)crec[i];
-        TS *p = v + ridx[i];
-        *p = (TS)((double)*p + x);
-    }
+    r.block(blockIdx.x);
 }
 
 // the imaging condition of two reverse steps in one pass over the gradient, for
@@ -155,6 +120,10 @@ __global__ void __launch_bounds__(256) k_imaging_pair(double *grad, const TS *mu
         }
     }
 }
+
+// steps from which the check of the sources and receivers (two small launches and
+// a wait, about 30 us) is worth the launch it saves on each step, 5 us
+constexpr int64_t END_LEAST_STEPS = 24;
 
 // sources up to which the imaging condition goes in pairs of steps
 constexpr int64_t PAIR_SRC_MAX = 4096;
@@ -207,12 +176,20 @@ static int imaging_pair(const hsx_grid *g, double *grad, const void *mu1, const 
     });
 }
 
-// one forward step: prev <- B(cur) step, source, record
+// One forward step: out <- B(cur) step, source, record.  work (NULL: never, else
+// step_end_check agreed): where end is set, the free surface of out, which the
+// next step begins with, goes with the sources and receivers in one launch;
+// *done says whether cur's was done like that, and on return whether out's was.
 static int fwd_step(const hsx_grid *g, const void *coef, const hsx_shot *sh, void *out, const void *prev, void *cur,
-                    int64_t n, void *traces, size_t es, hipStream_t s)
+                    int64_t n, void *traces, size_t es, const EndWork *work, bool end, bool *done, hipStream_t s)
 {
-    int rc = hsx_free_surface(g, cur, 0x3F, s);
+    int rc = *done ? HSX_OK : hsx_free_surface(g, cur, 0x3F, s);
     if (!rc) rc = hsx_ac2_step_to(g, out, prev, cur, coef, s);
+    *done = work && end;
+    if (!rc && *done)
+        return step_end_forward(g, out, sh->nsrc, sh->src_idx, (const char *)sh->wavelet + (size_t)n * sh->nsrc * es,
+                                sh->nrec, sh->rec_idx,
+                                traces && sh->nrec > 0 ? (char *)traces + (size_t)n * sh->nrec * es : nullptr, work, s);
     if (!rc && sh->nsrc > 0 && sh->nsrc <= SRCREC_MAX && sh->nrec > 0 && traces) {
         const int64_t nrec = sh->nrec;
         const unsigned nb = 1 + (unsigned)std::min<int64_t>((nrec + 255) / 256, 1024);
@@ -244,7 +221,7 @@ struct hsx_adjoint_plan {
     hsx_adjoint_opts opt;
     size_t es = 4, bytes = 0, snap = 0;
     int64_t nseg = 0;
-    hsx::Dev traces, res, crec, partial, msum, side, m1, m2, ck, fa, fb;
+    hsx::Dev traces, res, crec, partial, msum, side, end, m1, m2, ck, fa, fb;
     std::vector<hsx::Dev> q;   // wavefields q^{m}, m from the segment start - 1
 };
 
@@ -333,10 +310,17 @@ static int plan_run(hsx_adjoint_plan *P, const hsx_grid *g, const void *coef, co
 
     // ---- forward pass (traces only when the residual is formed here)
     void *tr = given_residual ? nullptr : P->traces.p;
+    bool merge = false, done = false;
+    if (nt >= END_LEAST_STEPS && (rc = step_end_check(g, sh->nsrc, sh->src_idx, nrec, sh->rec_idx, (EndWork *)P->end.p,
+                                                      &merge, s)))
+        return rc;
+    const EndWork *end = merge ? (const EndWork *)P->end.p : nullptr;
     if ((rc = zero(g, loc(-1), s)) || (rc = zero(g, loc(0), s))) return rc;
     for (int64_t n = 0; n < nt; n++) {
         if (K > 0 && !in_place && n % K == 0 && (rc = save(n / K, loc(n), loc(n - 1)))) return rc;
-        if ((rc = fwd_step(g, coef, sh, loc(n + 1), loc(n - 1), loc(n), n, tr, es, s))) return rc;
+        // (a 16-bit checkpoint holds the wavefield before its free surface)
+        const bool last = n + 1 == nt || (K > 0 && !in_place && (n + 1) % K == 0);
+        if ((rc = fwd_step(g, coef, sh, loc(n + 1), loc(n - 1), loc(n), n, tr, es, end, !last, &done, s))) return rc;
     }
 
     // ---- residual and misfit
@@ -374,12 +358,14 @@ static int plan_run(hsx_adjoint_plan *P, const hsx_grid *g, const void *coef, co
     // plain step 28.7).  hold: the first of a pair, imaged with the next step;
     // q_up: its latest wavefield, in the second one.
     const bool pairs = sh->nsrc <= PAIR_SRC_MAX;
+    bool bc_done = false;          // mu1's free surface went with the end of the step before
     auto back_step = [&](int64_t k, bool hold, const void *q_up, const void *qk, const void *qk1,
                          const void *qk2) -> int {
         // mu^k = 2 mu^{k+1} - (mu^{k+2} - c e^k) + c L mu^{k+1}: the residual
         // went into mu^{k+2} (mu2) before the step, so that the step's output is
         // mu^k complete and the imaging condition can be taken from it
-        int r = hsx_free_surface(g, mu1, 0x3F, s);
+        int r = bc_done ? HSX_OK : hsx_free_surface(g, mu1, 0x3F, s);
+        bc_done = false;
         if (!r) {
             r = fuse_img && !hold ? tiled_ac2_step_img(g, mu2, mu1, coef, grad, qk, qk1, qk2, q_up, rim, img_scale, s)
                                   : HSX_ERR_UNSUPPORTED;
@@ -396,16 +382,21 @@ static int plan_run(hsx_adjoint_plan *P, const hsx_grid *g, const void *coef, co
         if (!r && (ns > 0 || nr > 0)) {
             r = dispatch_types(g, [&](auto ts, auto) -> int {
                 using TS = decltype(ts);
-                const uint32_t nbs = (uint32_t)((ns + 255) / 256);
-                const uint32_t nbr = (uint32_t)std::min<int64_t>((nr + 255) / 256, 1024);
-                hipLaunchKernelGGL(k_imgsrc_residual<TS>, dim3(nbs + nbr), dim3(256), 0, s, grad, (const TS *)mu2,
-                                   (const TS *)qk, (const TS *)qk1, (const TS *)qk2,
-                                   hold || q_up ? (double *)P->side.p : (double *)nullptr, (int)hold, ns, sh->src_idx,
-                                   ns > 0 ? (const TS *)((const char *)sh->wavelet + (size_t)(k - 1) * ns * es)
-                                          : (const TS *)nullptr,
-                                   img_scale, rimb, g->n1, g->n1 * g->n2, nbs, (TS *)mu1, npoint, nr, sh->rec_idx,
-                                   nr > 0 ? (const TS *)res_at(k - 1) : (const TS *)nullptr, (const TS *)P->crec.p);
-                HSX_LAUNCHED("k_imgsrc_residual");
+                const ReverseEnd<TS> e = {
+                    grad, (const TS *)mu2, (const TS *)qk, (const TS *)qk1, (const TS *)qk2,
+                    hold || q_up ? (double *)P->side.p : (double *)nullptr, (int)hold, ns, sh->src_idx,
+                    ns > 0 ? (const TS *)((const char *)sh->wavelet + (size_t)(k - 1) * ns * es) : (const TS *)nullptr,
+                    img_scale, rimb, g->n1, g->n1 * g->n2, (uint32_t)((ns + 255) / 256),
+                    (uint32_t)std::min<int64_t>((nr + 255) / 256, 1024), (TS *)mu1, npoint, nr, sh->rec_idx,
+                    nr > 0 ? (const TS *)res_at(k - 1) : (const TS *)nullptr, (const TS *)P->crec.p};
+                // with the free surface of mu^k, which the next step reads
+                if (k >= 2) {
+                    const int r1 = step_end_reverse(g, mu2, e, s);
+                    bc_done = r1 == HSX_OK;
+                    if (r1 != HSX_ERR_UNSUPPORTED) return r1;
+                }
+                hipLaunchKernelGGL(k_reverse_end<TS>, dim3(e.nb_src + e.nb_rec), dim3(256), 0, s, e);
+                HSX_LAUNCHED("k_reverse_end");
                 return HSX_OK;
             });
         }
@@ -434,8 +425,11 @@ static int plan_run(hsx_adjoint_plan *P, const hsx_grid *g, const void *coef, co
             return q[m - n0 + 1].p;
         };
         if (!in_place && (rc = restore(seg, at(n0), at(n0 - 1)))) return rc;
-        for (int64_t n = n0; n < (in_place ? n1 - 2 : n1); n++)
-            if ((rc = fwd_step(g, coef, sh, at(n + 1), at(n - 1), at(n), n, nullptr, es, s))) return rc;
+        const int64_t ne = in_place ? n1 - 2 : n1;
+        done = false;
+        for (int64_t n = n0; n < ne; n++)
+            if ((rc = fwd_step(g, coef, sh, at(n + 1), at(n - 1), at(n), n, nullptr, es, end, n + 1 < ne, &done, s)))
+                return rc;
         if ((rc = reverse(n1, n0, at))) return rc;
     }
     double m = 0.0;
@@ -460,11 +454,19 @@ int hsx_forward(const hsx_grid *g, const void *coef, const hsx_shot *sh, void *t
     const size_t bytes = (size_t)(g->n1 * g->n2 * g->n3) * es;
     hipStream_t s = stream_of(stream);
     Dev a, b;
+    Dev work;
+    bool merge = false, done = false;
+    if (sh->nt >= END_LEAST_STEPS) {
+        if ((rc = work.alloc(sizeof(EndWork))) ||
+            (rc = step_end_check(g, sh->nsrc, sh->src_idx, sh->nrec, sh->rec_idx, (EndWork *)work.p, &merge, s)))
+            return rc;
+    }
+    const EndWork *end = merge ? (const EndWork *)work.p : nullptr;
     if ((rc = a.alloc(bytes)) || (rc = b.alloc(bytes))) return rc;
     if ((rc = zero(g, a.p, s)) || (rc = zero(g, b.p, s))) return rc;
     void *prev = a.p, *cur = b.p;
     for (int64_t n = 0; n < sh->nt; n++) {
-        if ((rc = fwd_step(g, coef, sh, prev, prev, cur, n, traces, es, s))) return rc;
+        if ((rc = fwd_step(g, coef, sh, prev, prev, cur, n, traces, es, end, n + 1 < sh->nt, &done, s))) return rc;
         std::swap(prev, cur);
     }
     HSX_HIP(hipStreamSynchronize(s));   // the buffers are freed on return
@@ -499,7 +501,7 @@ int hsx_adjoint_plan_create(const hsx_grid *g, int64_t nt, int64_t nrec, const h
     };
     if ((rc = P->traces.alloc(ntr * P->es)) || (rc = P->res.alloc(ntr * P->es)) || (rc = P->crec.alloc(nrec * P->es)) ||
         (rc = P->partial.alloc(4096 * sizeof(double))) || (rc = P->msum.alloc(sizeof(double))) ||
-        (rc = P->side.alloc(PAIR_SRC_MAX * sizeof(double))) ||
+        (rc = P->side.alloc(PAIR_SRC_MAX * sizeof(double))) || (rc = P->end.alloc(sizeof(EndWork))) ||
         (rc = P->m1.alloc(P->bytes)) || (rc = P->m2.alloc(P->bytes)))
         return bail(rc);
     P->q.resize((K == 0 ? nt : std::min(K, nt)) + 2);
