@@ -136,7 +136,7 @@ struct Dev {
     }
     int alloc(size_t bytes)
     {
-        hipError_t e = hipMalloc(&p, bytes ? bytes : 1);
+        hipError_t e = dev_malloc(&p, bytes);
         return e == hipSuccess ? HSX_OK : hip_fail(e, "hipMalloc (adjoint buffers)");
     }
     char *c() const { return (char *)p; }
@@ -453,23 +453,28 @@ int hsx_forward(const hsx_grid *g, const void *coef, const hsx_shot *sh, void *t
     const size_t es = g->storage == HSX_FP64 ? 8 : 4;
     const size_t bytes = (size_t)(g->n1 * g->n2 * g->n3) * es;
     hipStream_t s = stream_of(stream);
-    Dev a, b;
-    Dev work;
+    // both wavefields and the step ends' workspace
+    const size_t each = (bytes + 255) / 256 * 256;
+    struct Work {
+        WorkBuf b;
+        bool idle = false;
+        ~Work() { work_give(b, idle); }
+    } buf;
+    if ((rc = work_take(2 * each + sizeof(EndWork), &buf.b))) return rc;
+    void *prev = buf.b.p, *cur = (char *)prev + each;
+    EndWork *work = (EndWork *)((char *)cur + each);
     bool merge = false, done = false;
-    if (sh->nt >= END_LEAST_STEPS) {
-        if ((rc = work.alloc(sizeof(EndWork))) ||
-            (rc = step_end_check(g, sh->nsrc, sh->src_idx, sh->nrec, sh->rec_idx, (EndWork *)work.p, &merge, s)))
-            return rc;
-    }
-    const EndWork *end = merge ? (const EndWork *)work.p : nullptr;
-    if ((rc = a.alloc(bytes)) || (rc = b.alloc(bytes))) return rc;
-    if ((rc = zero(g, a.p, s)) || (rc = zero(g, b.p, s))) return rc;
-    void *prev = a.p, *cur = b.p;
+    if (sh->nt >= END_LEAST_STEPS &&
+        (rc = step_end_check(g, sh->nsrc, sh->src_idx, sh->nrec, sh->rec_idx, work, &merge, s)))
+        return rc;
+    const EndWork *end = merge ? work : nullptr;
+    if ((rc = zero(g, prev, s)) || (rc = zero(g, cur, s))) return rc;
     for (int64_t n = 0; n < sh->nt; n++) {
         if ((rc = fwd_step(g, coef, sh, prev, prev, cur, n, traces, es, end, n + 1 < sh->nt, &done, s))) return rc;
         std::swap(prev, cur);
     }
-    HSX_HIP(hipStreamSynchronize(s));   // the buffers are freed on return
+    HSX_HIP(hipStreamSynchronize(s));   // the buffer may serve another call after the return
+    buf.idle = true;
     return HSX_OK;
 }
 

@@ -88,7 +88,7 @@ namespace hsx {
 
 static int dalloc(hsx_batch *b, size_t bytes, void **p)
 {
-    hipError_t e = hipMalloc(p, bytes ? bytes : 1);
+    hipError_t e = dev_malloc(p, bytes);
     if (e != hipSuccess) return hip_fail(e, "hipMalloc (batch)");
     b->owned.push_back(*p);
     return HSX_OK;

@@ -586,7 +586,8 @@ struct NoExtra {
 // other receivers.  All other sources and receivers lie strictly inside the
 // boundary planes (step_end_check), so that no thread uses a point that another
 // one changes.  Against sources and receivers in a launch of their own before
-// the free surface's (4.6 + 6.0 us on 200^3 FP32 order 8): ENDFIG.
+// the free surface's (4.6 + 6.0 us on 200^3 FP32 order 8): 6.9 us, the
+// shot of 100 steps 4172 -> 3996 us.
 template <typename TS>
 struct ForwardEnd {
     int ns;

@@ -39,6 +39,88 @@ struct State {
 };
 static State g;
 
+// Buffers that calls have given back (work_give): at most WORK_SLOTS, WORK_BYTES
+// together, the oldest freed first; all are freed when the device changes or an
+// allocation fails.  Allocating and freeing the two wavefields of one shot cost
+// 0.4 ms (200^3 FP32, a shot of 100 steps 4.00 -> 3.58 ms).
+constexpr int WORK_SLOTS = 4;
+constexpr size_t WORK_BYTES = (size_t)512 << 20;
+static std::mutex g_work_mu;
+static WorkBuf g_work[WORK_SLOTS];       // oldest first, empty ones (p NULL) last
+static size_t g_work_bytes = 0;
+
+// (under g_work_mu) takes entry k out of the list
+static WorkBuf work_out(int k)
+{
+    const WorkBuf b = g_work[k];
+    for (int i = k; i + 1 < WORK_SLOTS; i++) g_work[i] = g_work[i + 1];
+    g_work[WORK_SLOTS - 1] = WorkBuf();
+    g_work_bytes -= b.bytes;
+    return b;
+}
+
+static bool work_drop(void)
+{
+    std::lock_guard<std::mutex> lk(g_work_mu);
+    const bool any = g_work[0].p != nullptr;
+    while (g_work[0].p) (void)hipFree(work_out(0).p);
+    return any;
+}
+
+hipError_t dev_malloc(void **ptr, size_t bytes)
+{
+    hipError_t e = hipMalloc(ptr, bytes ? bytes : 1);
+    if (e == hipErrorOutOfMemory && work_drop()) {
+        (void)hipGetLastError();
+        e = hipMalloc(ptr, bytes ? bytes : 1);
+    }
+    return e;
+}
+
+int work_take(size_t bytes, WorkBuf *out)
+{
+    int dev = -1;
+    HSX_HIP(hipGetDevice(&dev));
+    {
+        // the smallest that holds it, and is not four times as large
+        std::lock_guard<std::mutex> lk(g_work_mu);
+        int best = -1;
+        for (int k = 0; k < WORK_SLOTS && g_work[k].p; k++)
+            if (g_work[k].device == dev && g_work[k].bytes >= bytes && g_work[k].bytes / 4 <= bytes &&
+                (best < 0 || g_work[k].bytes < g_work[best].bytes))
+                best = k;
+        if (best >= 0) {
+            *out = work_out(best);
+            return HSX_OK;
+        }
+    }
+    void *p = nullptr;
+    const hipError_t e = dev_malloc(&p, bytes);
+    if (e != hipSuccess) return hip_fail(e, "hipMalloc (work buffers)");
+    out->p = p;
+    out->bytes = bytes;
+    out->device = dev;
+    return HSX_OK;
+}
+
+void work_give(const WorkBuf &b, bool idle)
+{
+    if (!b.p) return;
+    WorkBuf old[WORK_SLOTS + 1];
+    int n = 0;
+    if (!idle || b.bytes > WORK_BYTES) {
+        old[n++] = b;
+    } else {
+        std::lock_guard<std::mutex> lk(g_work_mu);
+        while (g_work[WORK_SLOTS - 1].p || g_work_bytes + b.bytes > WORK_BYTES) old[n++] = work_out(0);
+        int k = 0;
+        while (g_work[k].p) k++;
+        g_work[k] = b;
+        g_work_bytes += b.bytes;
+    }
+    for (int i = 0; i < n; i++) (void)hipFree(old[i].p);
+}
+
 static int init_locked(int device)
 {
     int n = 0;
@@ -48,6 +130,7 @@ static int init_locked(int device)
     if (g.ready && g.device == device) return HSX_OK;
     if (g.ready) {
         // switching device: drop the old device's resources
+        (void)work_drop();
         for (int i = 0; i < SCRATCH_SLOTS; i++) {
             if (g.scratch[i]) (void)hipFree(g.scratch[i]);
             g.scratch[i] = nullptr;
@@ -94,7 +177,7 @@ int scratch_get(int slot, size_t bytes, void **ptr)
             g.scratch_bytes[slot] = 0;
         }
         size_t sz = bytes < 4096 ? 4096 : bytes;
-        HSX_HIP(hipMalloc(&g.scratch[slot], sz));
+        HSX_HIP(dev_malloc(&g.scratch[slot], sz));
         g.scratch_bytes[slot] = sz;
     }
     *ptr = g.scratch[slot];
@@ -237,7 +320,7 @@ int hsx_malloc(void **ptr, size_t bytes)
     int rc = ensure_init();
     if (rc) return rc;
     *ptr = nullptr;
-    HSX_HIP(hipMalloc(ptr, bytes ? bytes : 1));
+    HSX_HIP(dev_malloc(ptr, bytes));
     return HSX_OK;
 }
 

@@ -102,3 +102,33 @@ def test_two_dimensions(capi):
     a, b = _run(capi, sh, src, rec, wav, 30), _run(capi, sh, src, rec, wav[:20], 20)
     assert np.abs(b).max() > 0
     _same(a[:20], b)
+
+
+def test_shots_on_two_threads(oracle, capi):
+    """shots of different sizes on two threads and streams, whose buffers serve
+    one call after another: each one's traces stay its own"""
+    import threading
+
+    import torch
+    jobs = []
+    for k, n in enumerate([(24, 20, 18), (61, 20, 18), (30, 25, 22), (24, 20, 18)]):
+        sh = make_shot(oracle, n, 8, nt=30, seed=40 + k, with_obs=False)
+        d = [_dev(capi, sh[x]) for x in ("src", "rec", "wavelet", "coef")]
+        tr = capi.DeviceArray(30 * len(sh["rec"]) * 4)
+        desc = capi.make_shot(30, sh["dt"], (d[0], len(sh["src"])), d[2], (d[1], len(sh["rec"])))
+        ref = oracle.forward(sh["o"], sh["coef"], sh["iv"], 30, sh["src"], sh["wavelet"], sh["rec"])
+        jobs.append((capi.hsx_grid(sh["p"]), d[3], desc, tr, ref, d))
+    streams = [torch.cuda.Stream() for _ in range(2)]
+
+    def work(i):
+        for _ in range(5):
+            for g, coef, desc, tr, _, _ in jobs[i::2]:
+                capi.forward(g, coef, desc, tr, stream=streams[i].cuda_stream)
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for _, _, _, tr, ref, _ in jobs:
+        _same(tr.download(np.float32).reshape(ref.shape), ref)
