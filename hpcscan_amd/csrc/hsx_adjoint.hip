@@ -298,14 +298,10 @@ static int plan_run(hsx_adjoint_plan *P, const hsx_grid *g, const void *coef, co
         return m & 1 ? P->fa.p : P->fb.p;
     };
     auto save = [&](int64_t seg, const void *cur, const void *prev) -> int {
-        int r = hsx_ckpt_encode((const float *)cur, nullptr, npoint, ck_at(seg, 0), fmt, s);
-        if (!r) r = hsx_ckpt_encode((const float *)cur, (const float *)prev, npoint, ck_at(seg, 1), fmt, s);
-        return r;
+        return ckpt_encode_pair((const float *)cur, (const float *)prev, npoint, ck_at(seg, 0), ck_at(seg, 1), fmt, s);
     };
     auto restore = [&](int64_t seg, void *cur, void *prev) -> int {
-        int r = hsx_ckpt_decode(ck_at(seg, 0), npoint, fmt, nullptr, (float *)cur, s);
-        if (!r) r = hsx_ckpt_decode(ck_at(seg, 1), npoint, fmt, (const float *)cur, (float *)prev, s);
-        return r;
+        return ckpt_decode_pair(ck_at(seg, 0), ck_at(seg, 1), npoint, fmt, (float *)cur, (float *)prev, s);
     };
 
     // ---- forward pass (traces only when the residual is formed here)

@@ -5,8 +5,10 @@
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "hsx_internal.h"
+#include "hsx_step_end.h"
 
 namespace hsx {
 
@@ -79,17 +81,33 @@ __device__ __forceinline__ float dec16(uint16_t c, int fmt)
     return __bfloat162float(__ushort_as_bfloat16(c));
 }
 
-// max |a - (b ? b : 0)| into hdr[1] (as float bits; values are >= 0 so the
-// unsigned order of the bits is the float order)
-__global__ void __launch_bounds__(256) k_ckpt_maxabs(const float *a, const float *b, int64_t n, unsigned *hdr_bits)
+// The kernels take 16 bytes of floats at a time, in grid-stride loops over the
+// groups, the last n % 4 values one by one; VEC: every buffer 16-byte aligned.
+// PAIR: the two snapshots of a pair in one launch, u_n into p0 and u_n - u_{n-1}
+// into p1, so that each wavefield is read once for the two.  Bound by memory;
+// 208^3 FP32, a pair, us: clear 4.0 (two snapshots one after the other: 8), max
+// 17 (51), encode 16 (24), decode 19 (45).
+struct alignas(8) Code4 {
+    uint16_t c[4];
+};
+typedef float Float4 __attribute__((ext_vector_type(4)));
+
+template <bool VEC, typename F4, typename F1>
+__device__ __forceinline__ void ckpt_loop(int64_t n, F4 &&four, F1 &&one)
 {
-    float m = 0.f;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const float v = b ? a[i] - b[i] : a[i];
-        m = fmaxf(m, fabsf(v));
-    }
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+    const int64_t ng = VEC ? n / 4 : 0;
+    for (int64_t i = t; i < ng; i += step) four(i);
+    for (int64_t i = 4 * ng + t; i < n; i += step) one(i);
+}
+
+// max |a - (b ? b : 0)| of the block into hdr[1] (as float bits; values are >= 0
+// so the unsigned order of the bits is the float order)
+__device__ __forceinline__ void ckpt_max(float m, unsigned *hdr_bits)
+{
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
     __shared__ float wm[4];
+    __syncthreads();
     if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = m;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -98,35 +116,106 @@ __global__ void __launch_bounds__(256) k_ckpt_maxabs(const float *a, const float
     }
 }
 
-__global__ void __launch_bounds__(256) k_ckpt_encode(const float *a, const float *b, int64_t n, char *packed, int fmt)
+template <bool PAIR, bool VEC>
+__global__ void __launch_bounds__(256) k_ckpt_maxabs(const float *a, const float *b, int64_t n, unsigned *h0,
+                                                     unsigned *h1)
 {
-    float *hdr = reinterpret_cast<float *>(packed);
-    const float maxabs = hdr[1];
-    const float scale = maxabs > 0.f ? maxabs / fmt_target(fmt) : 1.f;
-    const float inv = 1.f / scale;
-    uint16_t *code = reinterpret_cast<uint16_t *>(packed + CKPT_HEADER);
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const float v = b ? a[i] - b[i] : a[i];
-        code[i] = enc16(v * inv, fmt);
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) hdr[0] = scale;
+    float m = 0.f, d = 0.f;
+    auto value = [&](float x, float y) {
+        m = fmaxf(m, fabsf(PAIR || !b ? x : x - y));
+        if (PAIR) d = fmaxf(d, fabsf(x - y));
+    };
+    ckpt_loop<VEC>(
+        n,
+        [&](int64_t i) {
+            const Float4 x = reinterpret_cast<const Float4 *>(a)[i];
+            Float4 y = {};
+            if (b) y = reinterpret_cast<const Float4 *>(b)[i];
+#pragma unroll
+            for (int e = 0; e < 4; e++) value(x[e], y[e]);
+        },
+        [&](int64_t i) { value(a[i], b ? b[i] : 0.f); });
+    ckpt_max(m, h0);
+    if (PAIR) ckpt_max(d, h1);
 }
 
-// out = decoded (mode 0) or out = base - decoded (mode 1)
-__global__ void __launch_bounds__(256) k_ckpt_decode(const char *packed, int64_t n, int fmt, const float *base,
-                                                     float *out)
+__device__ __forceinline__ float ckpt_scale(const char *packed, int fmt)
 {
-    const float scale = reinterpret_cast<const float *>(packed)[0];
-    const uint16_t *code = reinterpret_cast<const uint16_t *>(packed + CKPT_HEADER);
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const float v = dec16(code[i], fmt) * scale;
-        out[i] = base ? base[i] - v : v;
+    const float maxabs = reinterpret_cast<const float *>(packed)[1];
+    return maxabs > 0.f ? maxabs / fmt_target(fmt) : 1.f;
+}
+
+template <bool PAIR, bool VEC>
+__global__ void __launch_bounds__(256) k_ckpt_encode(const float *a, const float *b, int64_t n, char *p0, char *p1,
+                                                     int fmt)
+{
+    const float s0 = ckpt_scale(p0, fmt), s1 = PAIR ? ckpt_scale(p1, fmt) : 1.f;
+    const float i0 = 1.f / s0, i1 = 1.f / s1;
+    uint16_t *c0 = reinterpret_cast<uint16_t *>(p0 + CKPT_HEADER), *c1 = reinterpret_cast<uint16_t *>(p1 + CKPT_HEADER);
+    ckpt_loop<VEC>(
+        n,
+        [&](int64_t i) {
+            const Float4 x = reinterpret_cast<const Float4 *>(a)[i];
+            Float4 y = {};
+            if (b) y = reinterpret_cast<const Float4 *>(b)[i];
+            Code4 u, v;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                u.c[e] = enc16((PAIR || !b ? x[e] : x[e] - y[e]) * i0, fmt);
+                if (PAIR) v.c[e] = enc16((x[e] - y[e]) * i1, fmt);
+            }
+            reinterpret_cast<Code4 *>(c0)[i] = u;
+            if (PAIR) reinterpret_cast<Code4 *>(c1)[i] = v;
+        },
+        [&](int64_t i) {
+            const float x = a[i], y = b ? b[i] : 0.f;
+            c0[i] = enc16((PAIR || !b ? x : x - y) * i0, fmt);
+            if (PAIR) c1[i] = enc16((x - y) * i1, fmt);
+        });
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        reinterpret_cast<float *>(p0)[0] = s0;
+        if (PAIR) reinterpret_cast<float *>(p1)[0] = s1;
     }
 }
 
-__global__ void k_ckpt_clear(unsigned *hdr_bits)
+// out = decoded, or base - decoded; PAIR: cur from p0 and cur - decoded p1 into out
+template <bool PAIR, bool VEC>
+__global__ void __launch_bounds__(256) k_ckpt_decode(const char *p0, const char *p1, int64_t n, int fmt,
+                                                     const float *base, float *cur, float *out)
 {
-    if (threadIdx.x < 2) hdr_bits[threadIdx.x] = 0u;
+    const float s0 = reinterpret_cast<const float *>(p0)[0], s1 = PAIR ? reinterpret_cast<const float *>(p1)[0] : 1.f;
+    const uint16_t *c0 = reinterpret_cast<const uint16_t *>(p0 + CKPT_HEADER);
+    const uint16_t *c1 = reinterpret_cast<const uint16_t *>(p1 + CKPT_HEADER);
+    ckpt_loop<VEC>(
+        n,
+        [&](int64_t i) {
+            const Code4 u = reinterpret_cast<const Code4 *>(c0)[i];
+            Code4 v = {};
+            Float4 y = {}, x, o;
+            if (PAIR) v = reinterpret_cast<const Code4 *>(c1)[i];
+            if (!PAIR && base) y = reinterpret_cast<const Float4 *>(base)[i];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                x[e] = dec16(u.c[e], fmt) * s0;
+                o[e] = PAIR ? x[e] - dec16(v.c[e], fmt) * s1 : base ? y[e] - x[e] : x[e];
+            }
+            if (PAIR) reinterpret_cast<Float4 *>(cur)[i] = x;
+            reinterpret_cast<Float4 *>(out)[i] = o;
+        },
+        [&](int64_t i) {
+            const float x = dec16(c0[i], fmt) * s0;
+            if (PAIR) {
+                cur[i] = x;
+                out[i] = x - dec16(c1[i], fmt) * s1;
+            } else {
+                out[i] = base ? base[i] - x : x;
+            }
+        });
+}
+
+__global__ void k_ckpt_clear(unsigned *h0, unsigned *h1)
+{
+    if (threadIdx.x < 2) (blockIdx.x ? h1 : h0)[threadIdx.x] = 0u;
 }
 
 static unsigned blocks_for(int64_t n)
@@ -139,6 +228,50 @@ static unsigned blocks_for(int64_t n)
 static unsigned blocks_for_max(int64_t n)
 {
     return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 512));
+}
+
+template <bool PAIR>
+static int ckpt_encode(const float *u, const float *u_prev, int64_t n, char *p0, char *p1, int format, hipStream_t s)
+{
+    const bool vec = ((uintptr_t)u | (uintptr_t)u_prev) % 16 == 0;
+    const int64_t items = vec ? (n + 3) / 4 : n;
+    unsigned *h0 = reinterpret_cast<unsigned *>(p0), *h1 = reinterpret_cast<unsigned *>(p1);
+    hipLaunchKernelGGL(k_ckpt_clear, dim3(PAIR ? 2 : 1), dim3(64), 0, s, h0, h1);
+    HSX_LAUNCHED("k_ckpt_clear");
+    auto go = [&](auto v) -> int {
+        constexpr bool VEC = decltype(v)::value;
+        hipLaunchKernelGGL((k_ckpt_maxabs<PAIR, VEC>), dim3(blocks_for_max(items)), dim3(256), 0, s, u, u_prev, n, h0, h1);
+        HSX_LAUNCHED("k_ckpt_maxabs");
+        hipLaunchKernelGGL((k_ckpt_encode<PAIR, VEC>), dim3(blocks_for(items)), dim3(256), 0, s, u, u_prev, n, p0, p1,
+                           format);
+        HSX_LAUNCHED("k_ckpt_encode");
+        return HSX_OK;
+    };
+    return vec ? go(std::true_type()) : go(std::false_type());
+}
+
+template <bool PAIR>
+static int ckpt_decode(const char *p0, const char *p1, int64_t n, int format, const float *base, float *cur, float *out,
+                       hipStream_t s)
+{
+    const bool vec = ((uintptr_t)base | (uintptr_t)cur | (uintptr_t)out) % 16 == 0;
+    const unsigned nb = blocks_for(vec ? (n + 3) / 4 : n);
+    if (vec)
+        hipLaunchKernelGGL((k_ckpt_decode<PAIR, true>), dim3(nb), dim3(256), 0, s, p0, p1, n, format, base, cur, out);
+    else
+        hipLaunchKernelGGL((k_ckpt_decode<PAIR, false>), dim3(nb), dim3(256), 0, s, p0, p1, n, format, base, cur, out);
+    HSX_LAUNCHED("k_ckpt_decode");
+    return HSX_OK;
+}
+
+int ckpt_encode_pair(const float *u, const float *u_prev, int64_t n, void *p0, void *p1, int format, hipStream_t s)
+{
+    return ckpt_encode<true>(u, u_prev, n, (char *)p0, (char *)p1, format, s);
+}
+
+int ckpt_decode_pair(const void *p0, const void *p1, int64_t n, int format, float *u, float *u_prev, hipStream_t s)
+{
+    return ckpt_decode<true>((const char *)p0, (const char *)p1, n, format, nullptr, u, u_prev, s);
 }
 
 } // namespace hsx
@@ -223,14 +356,7 @@ int hsx_ckpt_encode(const float *u, const float *u_prev, int64_t n, void *packed
     if ((uintptr_t)packed % 16) return fail(HSX_ERR_INVALID, "packed snapshot not 16-byte aligned");
     if ((rc = ensure_init())) return rc;
     hipStream_t s = stream_of(stream);
-    unsigned *hdr = reinterpret_cast<unsigned *>(packed);
-    hipLaunchKernelGGL(k_ckpt_clear, dim3(1), dim3(64), 0, s, hdr);
-    HSX_LAUNCHED("k_ckpt_clear");
-    hipLaunchKernelGGL(k_ckpt_maxabs, dim3(blocks_for_max(n)), dim3(256), 0, s, u, u_prev, n, hdr);
-    HSX_LAUNCHED("k_ckpt_maxabs");
-    hipLaunchKernelGGL(k_ckpt_encode, dim3(blocks_for(n)), dim3(256), 0, s, u, u_prev, n, (char *)packed, format);
-    HSX_LAUNCHED("k_ckpt_encode");
-    return HSX_OK;
+    return ckpt_encode<false>(u, u_prev, n, (char *)packed, (char *)packed, format, s);
 }
 
 int hsx_ckpt_decode(const void *packed, int64_t n, int format, const float *base, float *out, void *stream)
@@ -242,10 +368,7 @@ int hsx_ckpt_decode(const void *packed, int64_t n, int format, const float *base
     if ((uintptr_t)packed % 16) return fail(HSX_ERR_INVALID, "packed snapshot not 16-byte aligned");
     if ((rc = ensure_init())) return rc;
     hipStream_t s = stream_of(stream);
-    hipLaunchKernelGGL(k_ckpt_decode, dim3(blocks_for(n)), dim3(256), 0, s, (const char *)packed, n, format, base,
-                       out);
-    HSX_LAUNCHED("k_ckpt_decode");
-    return HSX_OK;
+    return ckpt_decode<false>((const char *)packed, (const char *)packed, n, format, base, nullptr, out, s);
 }
 
 } // extern "C"

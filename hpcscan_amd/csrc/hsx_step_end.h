@@ -96,6 +96,11 @@ int step_end_forward(const hsx_grid *g, void *u, int64_t nsrc, const int64_t *sr
 template <typename TS>
 int step_end_reverse(const hsx_grid *g, void *u, const ReverseEnd<TS> &r, hipStream_t s);
 
+// both snapshots of a 16-bit checkpoint (u in p0, u - u_prev in p1; the codes of
+// hsx_ckpt_encode, 16-byte aligned buffers), and back
+int ckpt_encode_pair(const float *u, const float *u_prev, int64_t n, void *p0, void *p1, int format, hipStream_t s);
+int ckpt_decode_pair(const void *p0, const void *p1, int64_t n, int format, float *u, float *u_prev, hipStream_t s);
+
 } // namespace hsx
 
 #endif
