@@ -1,7 +1,7 @@
 // Batched shots: many grids (one order and precision, any sizes) advanced
 // together, one launch of each kernel per time step for all of them:
-//   free surface of every shot (2 launches: n1 faces and mirrors, then the
-//   boundary planes), the fused Ac2 step of every shot
+//   free surface of every shot (one launch; two, n1 faces and mirrors, then the
+//   boundary planes, where a grid's faces need them), the fused Ac2 step of every shot
 //   (one k_tiled_batch launch over the tiles of all grids), then sources and
 //   receivers of every shot (one launch, one workgroup per shot).
 // The whole time loop can be captured once into a HIP graph and replayed.
@@ -10,6 +10,7 @@
 #include <functional>
 #include <vector>
 
+#include "hsx_step_end.h"
 #include "hsx_tiled.h"
 
 namespace hsx {
@@ -73,6 +74,9 @@ struct hsx_batch {
     void *n1 = nullptr;                        // N1Faces per shot (k_bc_n1), when n1_nh > 0
     int n1_nh = 0;                             // R / vector width
     int64_t n1_rows = 0;                       // largest number of rows of an n1 face
+    void *one = nullptr;                       // table of bc_one_batch_launch, if it serves every shot
+    int one_nh = 0;
+    uint32_t one_blocks = 0;
     void *sr[2] = {nullptr, nullptr};          // SrcRec per shot, per parity
     std::function<int(int, hipStream_t)> step; // batched fused step, per parity
     std::vector<void *> step_owned;            // device argument tables of step
@@ -347,7 +351,9 @@ static int batch_record(hsx_batch *b, hipStream_t s)
     HSX_LAUNCHED("k_zero_batch");
     for (int64_t n = 0; n < b->nt; n++) {
         const int p = (int)(n & 1);
-        int rc = b->n1_nh ? bc_batch_fs_launch(b->storage, ns, (void *const *)b->bc_fields[p], (const N1Faces *)b->n1,
+        int rc = b->one ? bc_one_batch_launch(b->storage, ns, (void *const *)b->bc_fields[p], b->one, b->one_nh,
+                                              b->one_blocks, s)
+                 : b->n1_nh ? bc_batch_fs_launch(b->storage, ns, (void *const *)b->bc_fields[p], (const N1Faces *)b->n1,
                                                b->n1_nh, b->n1_rows, (const FaceSet *)b->sets, b->most,
                                                b->most_plane, s)
                           : bc_batch_launch(b->storage, ns, (void *const *)b->bc_fields[p], (const FaceSet *)b->sets,
@@ -411,6 +417,9 @@ int hsx_batch_create(int nshots, const hsx_grid *grids, const void *const *coef,
         hsx_batch_destroy(b);
         return code;
     };
+    const size_t one_bytes = bc_one_batch_bytes();
+    std::vector<char> one(nshots * one_bytes);
+    bool one_ok = true;
     for (int s = 0; s < nshots; s++) {
         const hsx_grid &g = grids[s];
         const int64_t n = g.n1 * g.n2 * g.n3;
@@ -426,6 +435,13 @@ int hsx_batch_create(int nshots, const hsx_grid *grids, const void *const *coef,
         if (!closed) return bail(fail(HSX_ERR_UNSUPPORTED, "batch: shot %d too small for the two-launch boundary", s));
         b->most = std::max(b->most, most);
         b->most_plane = std::max(b->most_plane, most_plane);
+        int nh = 0;
+        uint32_t blocks = 0;
+        one_ok = one_ok && ((uintptr_t)A | (uintptr_t)B) % 16 == 0 &&
+                 bc_one_batch_fill(&g, A, sets[s], one.data() + s * one_bytes, &nh, &blocks) &&
+                 (s == 0 || nh == b->one_nh);
+        b->one_nh = nh;
+        b->one_blocks = std::max(b->one_blocks, blocks);
         // n1 faces in one 16-byte pass where they qualify; the rest stay with
         // the generic face kernels (the boundary-plane set zmask / zidx is kept)
         N1Faces &x = n1[s];
@@ -459,6 +475,7 @@ int hsx_batch_create(int nshots, const hsx_grid *grids, const void *const *coef,
         (rc = upload(b, np.data(), np.size() * sizeof(int64_t), &b->npoint)) ||
         (rc = upload(b, sets.data(), sets.size() * sizeof(FaceSet), &b->sets)))
         return bail(rc);
+    if (one_ok && (rc = upload(b, one.data(), one.size(), &b->one))) return bail(rc);
     if (b->n1_nh && (rc = upload(b, n1.data(), n1.size() * sizeof(N1Faces), &b->n1))) return bail(rc);
     for (int p = 0; p < 2; p++)
         if ((rc = upload(b, bcf[p].data(), nshots * sizeof(void *), &b->bc_fields[p])) ||

@@ -96,6 +96,15 @@ int step_end_forward(const hsx_grid *g, void *u, int64_t nsrc, const int64_t *sr
 template <typename TS>
 int step_end_reverse(const hsx_grid *g, void *u, const ReverseEnd<TS> &r, hipStream_t s);
 
+// the free surface of many grids in one launch: bytes of one grid's entry in the
+// device table; the entry (false: this grid needs several launches), with its
+// n1 halo groups and blocks; the launch over all entries, of one nh, with the
+// largest number of blocks
+size_t bc_one_batch_bytes(void);
+bool bc_one_batch_fill(const hsx_grid *g, const void *u, const FaceSet &fs, void *out, int *nh, uint32_t *blocks);
+int bc_one_batch_launch(int storage, int nshots, void *const *d_fields, const void *d_grids, int nh, uint32_t blocks,
+                        hipStream_t s);
+
 // both snapshots of a 16-bit checkpoint (u in p0, u - u_prev in p1; the codes of
 // hsx_ckpt_encode, 16-byte aligned buffers), and back
 int ckpt_encode_pair(const float *u, const float *u_prev, int64_t n, void *p0, void *p1, int format, hipStream_t s);
