@@ -36,6 +36,8 @@ int contract_mode(void);               // hsx_set_contract: 1 = contracted tiled
 
 // device scratch owned by the library (grown on demand, freed at exit)
 int scratch_get(int slot, size_t bytes, void **ptr);
+enum { SCRATCH_TABLES = 0, SCRATCH_PARTIALS = 1, SCRATCH_SLOTS = 4 };
+
 // device memory of a call that ends with its stream idle: taken from the buffers
 // of earlier calls or allocated; work_give keeps it for later ones (idle: no
 // launch uses it any more) within the bounds of hsx_runtime.hip, or frees it
@@ -48,7 +50,6 @@ int work_take(size_t bytes, WorkBuf *out);
 void work_give(const WorkBuf &b, bool idle);
 // hipMalloc; when it fails for lack of memory, once more without the buffers kept
 hipError_t dev_malloc(void **ptr, size_t bytes);
-enum { SCRATCH_TABLES = 0, SCRATCH_PARTIALS = 1, SCRATCH_RESULT = 2, SCRATCH_SLOTS = 4 };
 
 // ---- descriptor checks ----------------------------------------------------------
 int check_grid(const hsx_grid *g);
