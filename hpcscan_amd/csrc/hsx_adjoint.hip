@@ -65,15 +65,34 @@ __device__ __forceinline__ bool on_source(int64_t j, int64_t nsrc, const int64_t
     return false;
 }
 
+// A step out of place writes the inner points of its output only; outside them a
+// step in place leaves q^{n-1} as its free surface left it.  A receiver there
+// records that (hsx_forward's traces, whose steps are in place), so the point is
+// carried from prev, q^{n-1}, into the output, whose two next steps need it in
+// turn.  prev NULL: a step in place, nothing to carry.
+template <typename TS>
+struct Carry {
+    const TS *prev;
+    Box in;
+    int64_t n1, n12;
+
+    __device__ __forceinline__ bool at(int64_t j) const
+    {
+        if (!prev) return false;
+        const int64_t i3 = j / n12, i2 = (j - i3 * n12) / n1, i1 = j - i3 * n12 - i2 * n1;
+        return i1 < in.s1 || i1 > in.e1 || i2 < in.s2 || i2 > in.e2 || i3 < in.s3 || i3 > in.e3;
+    }
+};
+
 template <typename TS>
 __global__ void __launch_bounds__(256) k_srcrec(TS *u, int64_t npoint, int64_t nsrc, const int64_t *src, const TS *w,
-                                                int64_t nrec, const int64_t *rec, TS *tr)
+                                                int64_t nrec, const int64_t *rec, TS *tr, Carry<TS> c)
 {
     if (blockIdx.x == 0) {
         for (int64_t i = threadIdx.x; i < nsrc; i += blockDim.x) {
-            if ((uint64_t)src[i] >= (uint64_t)npoint) continue;
-            TS *p = u + src[i];
-            *p = (TS)((double)*p + 1.0 * (double)w[i]);
+            const int64_t j = src[i];
+            if ((uint64_t)j >= (uint64_t)npoint) continue;
+            u[j] = (TS)((double)(c.at(j) ? c.prev[j] : u[j]) + 1.0 * (double)w[i]);
         }
         __syncthreads();
         for (int64_t i = threadIdx.x; i < nrec; i += blockDim.x) {
@@ -85,7 +104,20 @@ __global__ void __launch_bounds__(256) k_srcrec(TS *u, int64_t npoint, int64_t n
     for (int64_t i = (int64_t)(blockIdx.x - 1) * blockDim.x + threadIdx.x; i < nrec;
          i += (int64_t)(gridDim.x - 1) * blockDim.x) {
         const int64_t j = rec[i];
-        if (!on_source(j, nsrc, src)) tr[i] = (uint64_t)j < (uint64_t)npoint ? u[j] : (TS)0;
+        if (on_source(j, nsrc, src)) continue;
+        const bool in = (uint64_t)j < (uint64_t)npoint;
+        if (in && c.at(j)) u[j] = c.prev[j];
+        tr[i] = in ? u[j] : (TS)0;
+    }
+}
+
+// the receivers' points carried alone, before sources that take a launch of their own
+template <typename TS>
+__global__ void __launch_bounds__(256) k_carry(TS *u, int64_t npoint, int64_t nrec, const int64_t *rec, Carry<TS> c)
+{
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nrec; i += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t j = rec[i];
+        if ((uint64_t)j < (uint64_t)npoint && c.at(j)) u[j] = c.prev[j];
     }
 }
 
@@ -190,22 +222,32 @@ static int fwd_step(const hsx_grid *g, const void *coef, const hsx_shot *sh, voi
         return step_end_forward(g, out, sh->nsrc, sh->src_idx, (const char *)sh->wavelet + (size_t)n * sh->nsrc * es,
                                 sh->nrec, sh->rec_idx,
                                 traces && sh->nrec > 0 ? (char *)traces + (size_t)n * sh->nrec * es : nullptr, work, s);
-    if (!rc && sh->nsrc > 0 && sh->nsrc <= SRCREC_MAX && sh->nrec > 0 && traces) {
-        const int64_t nrec = sh->nrec;
-        const unsigned nb = 1 + (unsigned)std::min<int64_t>((nrec + 255) / 256, 1024);
-        return dispatch_types(g, [&](auto ts, auto) -> int {
+    const bool record = sh->nrec > 0 && traces;
+    const bool one = sh->nsrc > 0 && sh->nsrc <= SRCREC_MAX;
+    if (!rc && record && (one || out != prev)) {
+        const int64_t nrec = sh->nrec, npoint = g->n1 * g->n2 * g->n3;
+        const unsigned nb = (unsigned)std::min<int64_t>((nrec + 255) / 256, 1024);
+        rc = dispatch_types(g, [&](auto ts, auto) -> int {
             using TS = decltype(ts);
-            hipLaunchKernelGGL(k_srcrec<TS>, dim3(nb), dim3(256), 0, s, (TS *)out, g->n1 * g->n2 * g->n3, sh->nsrc,
-                               sh->src_idx, (const TS *)((const char *)sh->wavelet + (size_t)n * sh->nsrc * es), nrec,
-                               sh->rec_idx, (TS *)((char *)traces + (size_t)n * nrec * es));
-            HSX_LAUNCHED("k_srcrec");
+            const Carry<TS> c = {out != prev ? (const TS *)prev : (const TS *)nullptr, box_of(g->inner), g->n1,
+                                 g->n1 * g->n2};
+            if (one) {
+                hipLaunchKernelGGL(k_srcrec<TS>, dim3(1 + nb), dim3(256), 0, s, (TS *)out, npoint, sh->nsrc, sh->src_idx,
+                                   (const TS *)((const char *)sh->wavelet + (size_t)n * sh->nsrc * es), nrec,
+                                   sh->rec_idx, (TS *)((char *)traces + (size_t)n * nrec * es), c);
+                HSX_LAUNCHED("k_srcrec");
+            } else {
+                hipLaunchKernelGGL(k_carry<TS>, dim3(nb), dim3(256), 0, s, (TS *)out, npoint, nrec, sh->rec_idx, c);
+                HSX_LAUNCHED("k_carry");
+            }
             return HSX_OK;
         });
+        if (one || rc) return rc;
     }
     if (!rc && sh->nsrc > 0)
         rc = hsx_inject(g, out, sh->nsrc, sh->src_idx, (const char *)sh->wavelet + (size_t)n * sh->nsrc * es, nullptr,
                         1.0, HSX_INJECT_ADD, s);
-    if (!rc && sh->nrec > 0 && traces)
+    if (!rc && record)
         rc = hsx_gather(g, out, sh->nrec, sh->rec_idx, (char *)traces + (size_t)n * sh->nrec * es, s);
     return rc;
 }
