@@ -381,7 +381,7 @@ static int plan_run(hsx_adjoint_plan *P, const hsx_grid *g, const void *coef, co
     void *mu1 = P->m1.p, *mu2 = P->m2.p;   // mu^{k+1}, mu^{k+2}
     // the imaging condition fused into the adjoint step's kernel where the
     // tiled kernels take the grid (exact arithmetic only), else its own pass
-    const bool fuse_img = kernel_family() != HSX_KERNEL_REF && !contract_mode() && tiled_pays(g);
+    const bool fuse_img = kernel_family() != HSX_KERNEL_REF && !contract_mode() && step_tiled(g);
     // the residual of step k - 1 goes into mu^{k+1}: for k = nt here, for the
     // others in the launch that ends reverse step k
     auto res_at = [&](int64_t k) { return P->res.c() + (size_t)(k - 1) * nrec * es; };

@@ -182,6 +182,8 @@ int tiled_laplacian(const hsx_grid *g, const void *u, void *w, hipStream_t s);
 int tiled_ac2_step_fma(const hsx_grid *g, void *out, const void *prn, const void *prc, const void *coef,
                        hipStream_t s);
 int tiled_laplacian_fma(const hsx_grid *g, const void *u, void *w, hipStream_t s);
+// the fused step, one thread per point (hsx_stencil.hip)
+int ac2_step_points(const hsx_grid *g, void *out, const void *prn, const void *prc, const void *coef, hipStream_t s);
 // the fused step in place on prn with grad += scale * new prn * (q0 - 2 q1 + q2)
 // over box (inside the inner points), in double (the adjoint's imaging condition);
 // q3 not NULL: grad += scale * prc * (q3 - 2 q0 + q1), the step before's, first

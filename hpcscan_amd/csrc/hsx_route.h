@@ -15,11 +15,22 @@ namespace hsx {
 // MB) 15.7 (step) against 9.5.
 constexpr int64_t TILED_LEAST_BYTES = 5200000;
 bool tile_shape_forced(void);   // hsx_set_tile asks for a shape (hsx_tiled_ac2.hip)
-inline bool tiled_pays(const hsx_grid *g)
+// the library's own choice, where no shape is asked for
+inline bool tiled_own(const hsx_grid *g)
 {
     // (the contracted arithmetic exists in the tiled kernels only)
-    if (kernel_family() == HSX_KERNEL_TILED || contract_mode() || tile_shape_forced()) return true;
+    if (kernel_family() == HSX_KERNEL_TILED || contract_mode()) return true;
     return g->n1 * g->n2 * g->n3 * (g->storage == HSX_FP64 ? 8 : 4) >= TILED_LEAST_BYTES;
+}
+inline bool tiled_pays(const hsx_grid *g)
+{
+    return tile_shape_forced() || tiled_own(g);
+}
+// the fused step: also where hsx_autotune found a tile shape faster than the own choice
+bool step_shape_tuned(const hsx_grid *g);   // hsx_tiled_ac2.hip
+inline bool step_tiled(const hsx_grid *g)
+{
+    return tiled_pays(g) || step_shape_tuned(g);
 }
 
 } // namespace hsx

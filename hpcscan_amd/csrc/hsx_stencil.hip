@@ -222,6 +222,29 @@ static int ref_grid(const Box &b, dim3 &grid)
     return HSX_OK;
 }
 
+int ac2_step_points(const hsx_grid *g, void *out, const void *prn, const void *prc, const void *coef, hipStream_t s)
+{
+    const Box b = box_of(g->inner);
+    dim3 grid;
+    const int rc = ref_grid(b, grid);
+    if (rc) return rc;
+    return dispatch_types(g, [&](auto ts, auto tc) -> int {
+        using TS = decltype(ts);
+        using TC = decltype(tc);
+        const Coefs<TC> c = make_coefs<TC>(g);
+        return dispatch_R(g->fd_order / 2, [&](auto rc_) -> int {
+            constexpr int R = decltype(rc_)::value;
+            return dispatch_dim(g->dim, [&](auto dc) -> int {
+                constexpr int DIM = decltype(dc)::value;
+                hipLaunchKernelGGL((k_ac2_ref<TS, TC, R, DIM>), grid, dim3(RX, RY), 0, s, (TS *)out,
+                                   (const TS *)prn, (const TS *)prc, (const TS *)coef, b, g->n1, g->n1 * g->n2, c);
+                HSX_LAUNCHED("k_ac2_ref");
+                return HSX_OK;
+            });
+        });
+    });
+}
+
 static int stencil_checks(const hsx_grid *g, std::initializer_list<std::pair<const void *, const char *>> ptrs)
 {
     int rc = check_grid(g);
@@ -337,32 +360,15 @@ int hsx_ac2_step_to(const hsx_grid *g, void *out, const void *prn, const void *p
     if (rc) return rc;
     if (prn == prc || out == prc) return fail(HSX_ERR_INVALID, "prn / out and prc must be different grids");
     hipStream_t s = stream_of(stream);
-    if (kernel_family() != HSX_KERNEL_REF && tiled_pays(g)) {
+    if (kernel_family() != HSX_KERNEL_REF && step_tiled(g)) {
         rc = tiled_ac2_step(g, out, prn, prc, coef, s);
         if (rc != HSX_ERR_UNSUPPORTED || kernel_family() == HSX_KERNEL_TILED) return rc;
     }
-    const Box b = box_of(g->inner);
-    dim3 grid;
     if (g->dim == 2 && kernel_family() != HSX_KERNEL_REF) {
         rc = run_plane<true>(g, out, prn, prc, coef, s);
         if (rc != HSX_ERR_UNSUPPORTED) return rc;
     }
-    if ((rc = ref_grid(b, grid))) return rc;
-    return dispatch_types(g, [&](auto ts, auto tc) -> int {
-        using TS = decltype(ts);
-        using TC = decltype(tc);
-        const Coefs<TC> c = make_coefs<TC>(g);
-        return dispatch_R(g->fd_order / 2, [&](auto rc_) -> int {
-            constexpr int R = decltype(rc_)::value;
-            return dispatch_dim(g->dim, [&](auto dc) -> int {
-                constexpr int DIM = decltype(dc)::value;
-                hipLaunchKernelGGL((k_ac2_ref<TS, TC, R, DIM>), grid, dim3(RX, RY), 0, s, (TS *)out,
-                                   (const TS *)prn, (const TS *)prc, (const TS *)coef, b, g->n1, g->n1 * g->n2, c);
-                HSX_LAUNCHED("k_ac2_ref");
-                return HSX_OK;
-            });
-        });
-    });
+    return ac2_step_points(g, out, prn, prc, coef, s);
 }
 
 int hsx_ac2_step_fs(const hsx_grid *g, void *prn, const void *prc, const void *coef, int face_mask, int fold,

@@ -103,6 +103,32 @@ bool tuned_shape(const hsx_grid *g, int mode, TileCfg *out)
     return true;
 }
 
+bool step_shape_tuned(const hsx_grid *g)
+{
+    TileCfg c;
+    return tuned_shape(g, MODE_AC2, &c) && (c.lx || c.by || c.chunk || c.flags);
+}
+
+// default_shape of a grid whose arrays lie in the caches, as hsx_set_tile takes it
+static TileCfg cached_shape(const hsx_grid *g)
+{
+    TileCfg c = {0, 0, 0, 0};
+    (void)dispatch_types(g, [&](auto ts, auto tc) -> int {
+        using TS = decltype(ts);
+        using TC = decltype(tc);
+        return dispatch_R(g->fd_order / 2, [&](auto rc_) -> int {
+            constexpr int R = decltype(rc_)::value;
+            c = default_shape<TS, TC, R, MODE_AC2>(g);
+            const int64_t w = c.lx * (16 / (int64_t)sizeof(TS));
+            const int64_t tiles = (g->inner[1] - g->inner[0] + w) / w * ((g->inner[3] - g->inner[2] + c.by) / c.by);
+            c.chunk = (int)chunk_one_round(g->inner[5] - g->inner[4] + 1, R, tiles, 2 * device_cus(), 4);
+            c.flags &= ~TILE_FILL;
+            return HSX_OK;
+        });
+    });
+    return c;
+}
+
 } // namespace hsx
 
 using namespace hsx;
@@ -140,8 +166,8 @@ extern "C" int hsx_autotune(const hsx_grid *g, int reps, int shape[4], float *be
     const int64_t N3 = g->inner[5] - g->inner[4] + 1;
     const int R = g->fd_order / 2;
     // candidates: lanes x rows, stream mode, halo ring, n3 chunk; the first is
-    // the library's own choice, so the shape kept is never slower than it in
-    // this sweep
+    // the library's own choice (on small grids one thread per point), so the
+    // shape kept is never slower than it in this sweep
     std::vector<TileCfg> cand = {
         {0, 0, 0, 0},
         {64, 16, 0, 0}, {64, 16, 0, HSX_TILE_NO_RING}, {64, 16, 0, HSX_TILE_CACHED},
@@ -153,14 +179,20 @@ extern "C" int hsx_autotune(const hsx_grid *g, int reps, int shape[4], float *be
     };
     TileCfg best = {0, 0, 0, 0};
     float best_t = 1e30f;
-    const bool wide = wide_tiles_fit(g);
+    const bool wide = wide_tiles_fit(g), tiled = tiled_own(g);
+    if (!tiled) cand.push_back(cached_shape(g));
     for (const TileCfg &c : cand) {
         if (c.lx == 128 && !wide) continue;      // would run another candidate's shape
-        rc = run_tiled_shape<MODE_AC2>(g, buf[0], buf[0], buf[1], buf[2], s, c);   // warm-up (and fit check)
+        const bool points = !tiled && &c == &cand[0];
+        auto step = [&] {
+            return points ? ac2_step_points(g, buf[0], buf[0], buf[1], buf[2], s)
+                          : run_tiled_shape<MODE_AC2>(g, buf[0], buf[0], buf[1], buf[2], s, c);
+        };
+        rc = step();                                                               // warm-up (and fit check)
         if (rc == HSX_ERR_UNSUPPORTED) continue;
         if (rc) break;
         (void)hipEventRecord(e0, s);
-        for (int k = 0; k < reps && !rc; k++) rc = run_tiled_shape<MODE_AC2>(g, buf[0], buf[0], buf[1], buf[2], s, c);
+        for (int k = 0; k < reps && !rc; k++) rc = step();
         (void)hipEventRecord(e1, s);
         if (rc) break;
         (void)hipEventSynchronize(e1);

@@ -124,9 +124,11 @@ int         hsx_get_contract(void);
 #define HSX_TILE_NO_RING 4
 int         hsx_set_tile(int lanes_n1, int rows_n2, int chunk_planes, int flags);
 /* Tile autotuner (no counterpart in the reference): times the candidate
- * shapes of the fused step on scratch grids of g's layout (reps launches each)
- * and keeps the fastest for g's layout, FD order and precisions; the fused
- * step on such grids then uses it unless hsx_set_tile forces a shape.  shape[4] (may be NULL) = lanes, rows, chunk, flags of the choice;
+ * shapes of the fused step, and the library's own choice (on small grids one
+ * thread per point), on scratch grids of g's layout (reps launches each) and
+ * keeps the fastest for g's layout, FD order and precisions; the fused step on
+ * such grids then uses it unless hsx_set_tile forces a shape.  shape[4] (may be
+ * NULL) = lanes, rows, chunk, flags of the choice, all 0 for the library's own;
  * *best_ms (may be NULL) its time per launch.  Allocates 3 grids while it runs. */
 int         hsx_autotune(const hsx_grid *g, int reps, int shape[4], float *best_ms);
 int         hsx_autotune_clear(void);

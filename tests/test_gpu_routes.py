@@ -1,0 +1,105 @@
+"""Which kernel a call runs: shapes asked for, tuned shapes, grids at the ends of
+the rules (run with -m gpu)."""
+import numpy as np
+import pytest
+
+from hpcscan_amd.layout import make_layout
+from tests.launches import launches
+from tests.shots import make_shot
+from tests.test_gpu_adjoint import _dev, _same, _shot_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def _step(capi, p, **kw):
+    """the launches of the fused step on zero grids of p"""
+    g = capi.hsx_grid(p, **kw)
+    prn, prc, coef = (capi.DeviceArray(p.npoint * (8 if p.fp64 else 4)) for _ in range(3))
+    for d in (prn, prc, coef):
+        capi.array_op(g, capi.HSX_ARRAY_FILL, d, val=0.0)
+    capi.sync()
+    return launches(capi, lambda s: capi.ac2_step(g, prn, prc, coef, stream=s))
+
+
+# below the tiled kernels' own range (the tuner keeps one thread per point or a
+# tile shape, whichever is faster) and in it
+TUNED = [((100, 100, 100), 8, "f32"), ((40, 36, 32), 8, "f32"), ((60, 60, 60), 8, "f32"), ((128, 120, 110), 8, "f32"),
+         ((80, 70, 70), 8, "f64"), ((40, 36, 32), 8, "f64"), ((72, 62, 62), 16, "f64"), ((32, 32, 32), 16, "f64"),
+         ((96, 90, 90), 8, "f32c64"), ((88, 80, 80), 16, "f32c64"), ((88, 90, 80), 16, "f32"), ((32, 32, 32), 16, "f32")]
+
+
+@pytest.mark.parametrize("n,order,prec", TUNED)
+def test_step_runs_what_the_tuner_reports(capi, n, order, prec):
+    """the step on a tuned grid runs the shape that hsx_autotune returned, the
+    one that its time is of; 0, 0, 0, 0 is what the step runs untuned"""
+    p = make_layout(3, n, order, fp64=prec == "f64")
+    kw = {"compute_fp64": prec != "f32"}
+    capi.autotune_clear()
+    try:
+        own = _step(capi, p, **kw)
+        shape, ms = capi.autotune(capi.hsx_grid(p, **kw), reps=20)
+        print(f"n={n} order={order} {prec}: own {own}, tuned {shape} {1e3 * ms:.2f} us", flush=True)
+        tuned = _step(capi, p, **kw)
+        capi.autotune_clear()
+        lanes, rows, chunk, flags = shape
+        capi.set_tile(lanes, chunk, rows, flags)
+        assert tuned == _step(capi, p, **kw)
+    finally:
+        capi.set_tile(0, 0)
+        capi.autotune_clear()
+    assert _step(capi, p, **kw) == own
+
+
+def test_tuned_time_is_the_steps(capi):
+    """32 points an axis, order 16: a launch of any tile shape lasts three times
+    as long as one thread per point; the tuner's time is that of the step"""
+    import ctypes
+    p = make_layout(3, (32, 32, 32), 16)
+    g = capi.hsx_grid(p)
+    prn, prc, coef = (_dev(capi, np.zeros(p.npoint, np.float32)) for _ in range(3))
+    stream, e0, e1, ms = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_float()
+    L = capi.lib()
+    capi.check(L.hsx_stream_create(ctypes.byref(stream)))
+    for e in (e0, e1):
+        capi.check(L.hsx_event_create(ctypes.byref(e)))
+    capi.autotune_clear()
+    try:
+        told = min(capi.autotune(g, reps=50)[1] for _ in range(3))
+        ran = []
+        for _ in range(5):
+            capi.ac2_step(g, prn, prc, coef, stream=stream)
+            capi.check(L.hsx_event_record(e0, stream))
+            for _ in range(50):
+                capi.ac2_step(g, prn, prc, coef, stream=stream)
+            capi.check(L.hsx_event_record(e1, stream))
+            capi.sync(stream)
+            capi.check(L.hsx_event_elapsed_ms(e0, e1, ctypes.byref(ms)))
+            ran.append(ms.value / 50)
+    finally:
+        capi.autotune_clear()
+        for e in (e0, e1):
+            capi.check(L.hsx_event_destroy(e))
+        capi.check(L.hsx_stream_destroy(stream))
+    print(f"tuner {1e3 * told:.2f} us, step {1e3 * min(ran):.2f} us", flush=True)
+    # (the step may be bound by this loop's launches)
+    assert told < 2 * min(ran)
+
+
+def test_plan_with_a_tuned_shape_bit_exact(oracle, capi):
+    """a plan made with HSX_ADJ_AUTOTUNE on a grid below the tiled kernels' own
+    range, whose forward and reverse steps run the tuned shape"""
+    sh = make_shot(oracle, (72, 62, 62), 16, nt=25, fp64=True, seed=38)
+    g = capi.hsx_grid(sh["p"])
+    d, s = _shot_dev(capi, sh)
+    capi.autotune_clear()
+    try:
+        plan = capi.AdjointPlan(g, sh["nt"], len(sh["rec"]), 6, capi.HSX_CKPT_FP32, autotune=True)
+        grad = _dev(capi, np.zeros(sh["p"].npoint))
+        plan.gradient(g, d["coef"], s, _dev(capi, sh["d_obs"]), grad)
+        plan.close()
+    finally:
+        capi.autotune_clear()
+    gref, _ = oracle.gradient(sh["o"], sh["coef"], sh["iv"], sh["dt"], sh["nt"], sh["src"], sh["wavelet"],
+                              sh["rec"], sh["d_obs"])
+    assert np.abs(gref).max() > 0
+    _same(grad.download(np.float64), gref)
