@@ -20,6 +20,8 @@ inline bool tiled_own(const hsx_grid *g)
 {
     // (the contracted arithmetic exists in the tiled kernels only)
     if (kernel_family() == HSX_KERNEL_TILED || contract_mode()) return true;
+    // one thread per point has a plane per workgroup along z: 65535 at most
+    if (g->inner[5] - g->inner[4] >= 65535) return true;
     return g->n1 * g->n2 * g->n3 * (g->storage == HSX_FP64 ? 8 : 4) >= TILED_LEAST_BYTES;
 }
 inline bool tiled_pays(const hsx_grid *g)

@@ -7,6 +7,7 @@ from hpcscan_amd.layout import make_layout
 from tests.launches import launches
 from tests.shots import make_shot
 from tests.test_gpu_adjoint import _dev, _same, _shot_dev
+from tests.test_gpu_parity import PRECS, _layouts, _rand
 
 pytestmark = pytest.mark.gpu
 
@@ -103,3 +104,32 @@ def test_plan_with_a_tuned_shape_bit_exact(oracle, capi):
                               sh["rec"], sh["d_obs"])
     assert np.abs(gref).max() > 0
     _same(grad.download(np.float64), gref)
+
+
+@pytest.mark.parametrize("n3", [65535, 65536, 70000])
+def test_more_planes_than_one_launch_of_points(oracle, capi, n3):
+    """a small array (4.5 MB) of more than 65535 planes, which only the tiled
+    kernels take: step, Laplacian, D2 and D1 equal the oracle's"""
+    dtype, c64 = PRECS["f32"]
+    p, o = _layouts(oracle, 3, (2, 2, n3), 2, dtype, offset=(0, 0, 0))
+    assert p.n1 == p.n2 == 4
+    rng = np.random.default_rng(n3)
+    g = capi.hsx_grid(p, compute_fp64=c64)
+    u, coef, prn, w0 = (_rand(rng, p.npoint, dtype) for _ in range(4))
+    iv, iv1 = oracle.inv2(p.d, dtype, compute64=c64), oracle.inv1(p.d, dtype, compute64=c64)
+    du, dc, dp, dw = (_dev(capi, x) for x in (u, coef, prn, w0))
+    ref = prn.copy()
+    oracle.pressure_fd(o, ref, u, coef, iv, compute64=c64)
+    capi.ac2_step(g, dp, du, dc)
+    _same(dp.download(dtype), ref)
+    ref = w0.copy()
+    oracle.laplacian(o, u, ref, iv, compute64=c64)
+    capi.laplacian(g, du, dw)
+    _same(dw.download(dtype), ref)
+    for axis in range(3):
+        for op, ref_op, x in ((capi.fd_d2, oracle.fd_d2, iv), (capi.fd_d1, oracle.fd_d1, iv1)):
+            ref = w0.copy()
+            ref_op(o, axis, u, ref, x, compute64=c64)
+            dw.upload(w0)
+            op(g, axis, du, dw)
+            _same(dw.download(dtype), ref)
