@@ -1186,8 +1186,17 @@ inline int run_tiled_shape(const hsx_grid *g, void *out, const void *prn_in, con
         return dispatch_R(R, [&](auto rc_) -> int {
             constexpr int RR = decltype(rc_)::value;
             TileCfg cfg = cfg_in;
-            const bool none = cfg.lx == 0 && cfg.by == 0 && cfg.chunk == 0 && cfg.flags == 0;
-            if (!FOLD && none) cfg = default_shape<TS, TC, RR, MODE>(g);
+            if (!FOLD && cfg.lx == 0 && cfg.by == 0) {
+                // the chunk and the flags asked for, if any, on the library's own tile
+                const TileCfg own = default_shape<TS, TC, RR, MODE>(g);
+                cfg.lx = own.lx;
+                cfg.by = own.by;
+                if (cfg.flags == 0) cfg.flags = own.flags & ~TILE_FILL;
+                if (cfg.chunk == 0) {
+                    cfg.chunk = own.chunk;
+                    cfg.flags |= own.flags & TILE_FILL;
+                }
+            }
             int lx = pick_lx(g, VW, cfg, MODE == MODE_LAP);
             // the order-8 Laplacian drops the halo ring, whose halo rows still meet
             // in L2 with two streams instead of four (1000^3 1.84 / 1.88 ms, 800^3

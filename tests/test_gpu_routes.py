@@ -133,3 +133,34 @@ def test_more_planes_than_one_launch_of_points(oracle, capi, n3):
             dw.upload(w0)
             op(g, axis, du, dw)
             _same(dw.download(dtype), ref)
+
+
+# one grid of each of the step's own tiles: 128 x 8 with the ring, 64 x 8 in the
+# caches, 32 x 16 FP64, 32 x 8 with 12-plane chunks
+@pytest.mark.parametrize("n,order,prec,flags", [((508, 270, 130), 8, "f32", 1), ((128, 120, 110), 8, "f32", 6),
+                                                ((260, 240, 200), 8, "f64", 6), ((280, 260, 250), 8, "f32c64", 6)])
+def test_a_partly_given_shape_keeps_the_own_tile(capi, n, order, prec, flags):
+    """only a chunk or only flags asked for: lanes, rows and what else is left 0
+    stay the library's choice, and results the same"""
+    p = make_layout(3, n, order, fp64=prec == "f64")
+    kw = {"compute_fp64": prec != "f32"}
+    g = capi.hsx_grid(p, **kw)
+    rng = np.random.default_rng(5)
+    u, coef, prn = (rng.random(p.npoint, dtype=p.dtype) for _ in range(3))
+    du, dc, dp = (_dev(capi, x) for x in (u, coef, prn))
+    got = []
+    try:
+        for chunk, fl in ((0, 0), (20, 0), (0, flags)):
+            capi.set_tile(0, chunk, 0, fl)
+            (run,) = _step(capi, p, **kw)
+            dp.upload(prn)
+            capi.ac2_step(g, dp, du, dc)
+            got.append((run, dp.download(p.dtype)))
+            print(f"n={n} {prec} chunk {chunk} flags {fl}: {run}", flush=True)
+    finally:
+        capi.set_tile(0, 0)
+    own, chunked, flagged = (x[0] for x in got)
+    assert chunked[1:] == own[1:]              # threads and LDS bytes of the tile
+    assert flagged == own                      # flags: the own choice of the ring, other streams
+    for x in got[1:]:
+        _same(x[1], got[0][1])
