@@ -150,7 +150,7 @@ static int batch_setup_shape(hsx_batch *b, const hsx_grid *grids, const void *co
     // argument tables of this step; those of the step it replaces are freed
     std::vector<void *> mine;
     auto up = [&](const void *host, size_t bytes, void **p) -> int {
-        hipError_t e = hipMalloc(p, bytes ? bytes : 1);
+        hipError_t e = dev_malloc(p, bytes);
         if (e != hipSuccess) return hip_fail(e, "hipMalloc (batch step)");
         mine.push_back(*p);
         HSX_HIP(hipMemcpy(*p, host, bytes, hipMemcpyHostToDevice));
@@ -246,7 +246,7 @@ static int batch_setup_persistent(hsx_batch *b, const hsx_grid *grids, const voi
         return fail(HSX_ERR_INVALID, "batch: %lld of %lld parts cut", (long long)g, (long long)parts);
     std::vector<void *> mine;
     auto up = [&](const void *host, size_t bytes, void **p) -> int {
-        hipError_t e = hipMalloc(p, bytes ? bytes : 1);
+        hipError_t e = dev_malloc(p, bytes);
         if (e != hipSuccess) return hip_fail(e, "hipMalloc (batch step)");
         mine.push_back(*p);
         HSX_HIP(hipMemcpy(*p, host, bytes, hipMemcpyHostToDevice));

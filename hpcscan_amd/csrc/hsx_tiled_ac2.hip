@@ -151,7 +151,7 @@ extern "C" int hsx_autotune(const hsx_grid *g, int reps, int shape[4], float *be
             if (p) (void)hipFree(p);
     };
     for (void *&p : buf) {
-        hipError_t e = hipMalloc(&p, bytes);
+        hipError_t e = dev_malloc(&p, bytes);
         if (e != hipSuccess) {
             release();
             return hip_fail(e, "hipMalloc (autotune)");
