@@ -68,6 +68,7 @@ SIGNATURES = {
     "hsx_device_info": (_i, [_i, _P(HsxDeviceProps)]),
     "hsx_malloc": (_i, [_P(_vp), _sz]),
     "hsx_free": (_i, [_vp]),
+    "hsx_release_buffers": (_i, []),
     "hsx_memcpy_h2d": (_i, [_vp, _vp, _sz, _vp]),
     "hsx_memcpy_d2h": (_i, [_vp, _vp, _sz, _vp]),
     "hsx_memcpy_d2d": (_i, [_vp, _vp, _sz, _vp]),
@@ -347,6 +348,11 @@ def min_max(g: HsxGrid, u, r, stream=None):
     out = (ctypes.c_double * 2)()
     check(lib().hsx_min_max(ctypes.byref(g), dptr(u), rng(r), out, stream))
     return out[0], out[1]
+
+
+def release_buffers():
+    """Give back the device memory kept from finished shots (hsx_release_buffers)."""
+    check(lib().hsx_release_buffers())
 
 
 def sync(stream=None):

@@ -83,6 +83,13 @@ int         hsx_device_count(int *count);
 int         hsx_device_info(int device, hsx_device_props *out);
 int         hsx_malloc(void **ptr, size_t bytes);
 int         hsx_free(void *ptr);
+/* Gives back the device memory that the library keeps from finished calls for
+ * the next ones: the wavefields of hsx_forward, at most 4 buffers and 512 MiB
+ * together (a larger one is freed when its call ends).  Without this call they
+ * are freed when hsx_init changes the device and when an allocation of the
+ * library would fail; an allocator beside it (PyTorch's) cannot reclaim them.
+ * Buffers of calls that are running on other threads are not touched. */
+int         hsx_release_buffers(void);
 int         hsx_memcpy_h2d(void *dst, const void *src, size_t bytes, void *stream);
 int         hsx_memcpy_d2h(void *dst, const void *src, size_t bytes, void *stream);
 int         hsx_memcpy_d2d(void *dst, const void *src, size_t bytes, void *stream);
@@ -268,6 +275,8 @@ typedef struct {
     const int64_t *rec_idx;
 } hsx_shot;
 
+/* Returns after the stream has finished; keeps its two wavefields for the next
+ * call (hsx_release_buffers). */
 int hsx_forward(const hsx_grid *g, const void *coef, const hsx_shot *shot, void *traces, void *stream);
 
 /* d_obs is the residual itself (the adjoint source, e.g. the gradient of any
