@@ -777,11 +777,12 @@ __global__ void __launch_bounds__(LX *BY) k_tiled_batch_seg(const TiledArgs<TC> 
 // BY rows along n2, chunk = planes per workgroup along n3, streams = cached or
 // nontemporal prn / coef / output, halo ring on or off.  hsx_set_tile()
 // overrides each of them (0 = the choice made here):
-//  * BY = 16 with the halo ring where its LDS fits (LX >= 32), else BY = 8;
+//  * default_shape: grids that lie in the caches, and the step on larger ones;
+//  * else BY = 16 with the halo ring where its LDS fits (LX >= 32), else BY = 8;
 //  * 16-row tiles: one chunk per tile when the tiles fill the device once
 //    (every workgroup starts together, so tiles that share halo rows stream
 //    through L2 in step), nontemporal streams;
-//  * 8-row tiles: short chunks, cached streams.
+//  * 8-row tiles: short chunks, cached streams, where default_shape says nothing.
 struct TileCfg {
     int lx, by, chunk, flags;
 };
@@ -806,21 +807,31 @@ struct ImgReq {
 };
 extern thread_local ImgReq t_img;     // defined in hsx_tiled_ac2_img.hip
 constexpr int TILE_LDS_MAX = 163840;  // gfx950: 160 KiB of LDS per workgroup
-// internal flag of a shape: chunks that give one round of two workgroups per CU,
+// internal flag of a shape: chunks that give one round of fill_slots workgroups,
 // down to 4 planes (grids that lie in the caches, default_shape)
 constexpr int TILE_FILL = 256;
 
-// lanes of the widest tile: 64, or 16 / 32 where they hold the row.  The
-// Laplacian on large grids takes 32 where tiles of 64 span more than 5/4 of the
-// width of tiles of 32 (320^3 order 8 61.6 against 68 us); the widths are fitted
-// to the row afterwards (tile_lanes), and the other kernels do as well or
-// better with the wider tiles (D2 of 320^3 42-44 us against 47-51).
+// first n1 index of the tiles: vectors counted back from the row's end, so that
+// none reaches past it; a multiple of vw where n1 is one, else down to -(vw - 1)
+inline int64_t tiles_start(const hsx_grid *g, int vw)
+{
+    return g->inner[0] - (g->inner[0] + vw - g->n1 % vw) % vw;
+}
+
+// lanes of the widest tile: 64, or 16 / 32 where they hold the row (with what its
+// first vector takes in before it: 64 points may be 17 vectors).  narrow: 32
+// also where tiles of 64 span more than 5/4 of the width of tiles of 32: the
+// Laplacian (320^3 order 8 61.6 against 68 us), the FP32 step (320^3 order 12 119
+// against 139), D2 and D1 along n1 and n2 from order 10 on, with FP64 compute from
+// order 6 on (320^3 order 12 44 against 55, with FP64 compute 53 against 71).  The
+// widths are fitted to the row afterwards (tile_lanes), and the others do as well
+// or better with the wider tiles (FP32 D2 of 320^3 at order 8 39 us against 53).
 inline int pick_lx(const hsx_grid *g, int vw, const TileCfg &cfg, bool narrow = false)
 {
     if (cfg.lx) return cfg.lx;
-    const int64_t N1 = g->inner[1] - g->inner[0] + 1;
-    if (N1 <= 16 * vw) return 16;
-    if (N1 <= 32 * vw) return 32;
+    const int64_t N1 = g->inner[1] - g->inner[0] + 1, span = g->inner[1] - tiles_start(g, vw) + 1;
+    if (span <= 16 * vw) return 16;
+    if (span <= 32 * vw) return 32;
     const int64_t w64 = (N1 + 64 * vw - 1) / (64 * vw) * (64 * vw);
     const int64_t w32 = (N1 + 32 * vw - 1) / (32 * vw) * (32 * vw);
     return narrow && 4 * w64 > 5 * w32 ? 32 : 64;
@@ -879,6 +890,36 @@ inline int tile_lanes(int64_t span1, int ntx)
     if (ntx > 1) lx = (lx + 7) / 8 * 8;
     lx = std::max(lx, std::max(8, 2 * NHG));
     return 8 * lx <= 7 * LX ? lx : LX;
+}
+
+// the arrays of a launch, which the rules below look at
+template <typename TS, int MODE>
+inline int64_t shape_bytes(const hsx_grid *g)
+{
+    return g->n1 * g->n2 * g->n3 * (int64_t)sizeof(TS) * (mode_ac2(MODE) ? 3 : 2);
+}
+
+// Workgroups of the one round of TILE_FILL: two per CU, and as many more as it
+// takes to have fill_threads threads on each.  Tiles of 16 lanes have 128 threads,
+// narrow rows fitted by tile_lanes as few as 64: two of these leave a CU with two
+// waves (FP32, us, two workgroups per CU -> 1024 threads: order 8 64 x 300 x 500
+// Laplacian 36 -> 22, order 4 60 x 60 x 1000 step 18.3 -> 12.3, order 12 280^3 D2
+// along n2 55 -> 37).  More threads mean shorter chunks, which load 2R planes more
+// each: the FP64 step (its planes are twice as large) and D2 / D1 along n3 (nothing
+// but planes) keep 512 where that costs more, all of FP64 along n3 from order 4 on
+// (250 x 120 x 333 order 8 26 against 35 us with 1024), FP32 above 120 MB
+// (280 x 224 x 283 order 8 25 against 30).
+template <typename TS, int R, int MODE>
+inline int fill_threads(int64_t bytes)
+{
+    constexpr bool FP64 = sizeof(TS) == 8;
+    if (MODE == MODE_AC2_IMG || (FP64 && mode_ac2(MODE))) return 512;
+    if (MODE == MODE_D2Z || MODE == MODE_D1Z) return (FP64 ? R == 1 : bytes <= 120000000) ? 1024 : 512;
+    return 1024;
+}
+inline int64_t fill_slots(int threads, int cu_threads)
+{
+    return (int64_t)device_cus() * std::max(2, cu_threads / threads);
 }
 
 // resident workgroups per CU of a kernel instance (once per instantiation;
@@ -946,9 +987,7 @@ inline int fill_tiled_args(const hsx_grid *g, void *out, const void *prn_in, con
     a.e2 = g->inner[3];
     a.s3 = g->inner[4];
     a.e3 = g->inner[5];
-    // vectors counted back from the row's end, so that none reaches past it; a
-    // multiple of VW where n1 is one, else down to -(VW - 1)
-    a.t1s = a.s1 - (a.s1 + VW - a.n1 % VW) % VW;
+    a.t1s = tiles_start(g, VW);
     const int64_t span1 = a.e1 - a.t1s + 1;
     a.ntx = (int)((span1 + LX * VW - 1) / (LX * VW));
     a.lx = tile_lanes<R, VW, LX>(span1, a.ntx);
@@ -959,7 +998,7 @@ inline int fill_tiled_args(const hsx_grid *g, void *out, const void *prn_in, con
     const int64_t cs = STREAM && cfg.chunk <= 0 && chunk <= 0 && !(cfg.flags & TILE_FILL) ? chunk_stream(N3, R, tiles, LX * BY) : 0;
     const int64_t len = cfg.chunk > 0 ? std::min<int64_t>(cfg.chunk, N3)
                         : (cfg.flags & TILE_FILL)
-                            ? chunk_one_round(N3, R, tiles, std::min<int64_t>(slots, 2 * device_cus()), 4)
+                            ? chunk_one_round(N3, R, tiles, std::min(slots, fill_slots(a.lx * BY, fill_threads<TS, R, MODE>(shape_bytes<TS, MODE>(g)))), 4)
                         : chunk > 0           ? std::min<int64_t>(std::max<int64_t>(chunk, 4 * R), N3)
                         : cs > 0              ? cs
                         : (BY == 16 || RING) ? chunk_one_round(N3, R, tiles, slots)
@@ -1106,39 +1145,51 @@ inline bool wide_by_default(const hsx_grid *g)
 // and fill_tiled_args).  All figures: kernel alone, us, 'was' = 16-row tiles
 // with the ring in chunks of at least 4R planes, or 64 x 8 for FP64 values.
 //
-// Grids whose arrays lie in the 256 MB Infinity Cache together (up to 200 MB)
-// are bound by the planes a workgroup streams one after the other and by CUs
-// without work, not by bytes: 8-row tiles without the ring (several workgroups
-// per CU), chunks of 4 planes or more that give one round of two workgroups per
-// CU, cached streams (the step; the kernels that write a second grid and never
-// read it again keep nontemporal ones).  Step, FP32 order 8: 128^3 8.4 (was
-// 21), 160^3 16 (27), 200^3 28.5 (39), order 16 37 (56); FP64 150^3 25 (31);
-// FP32 storage with FP64 compute 200^3 31 (41); Laplacian 160^3 12.4 (21), 256^3
-// order 12 46 (61); D2 of 160^3 8.2-8.5 (12-13).  32 lanes from order 10 on and
-// for FP64 values, which keep twice the registers (200^3 order 12 34 against 37).
+// Grids whose arrays lie in the 256 MB Infinity Cache together are bound by the
+// planes a workgroup streams one after the other and by CUs without work, not by
+// bytes: 8-row tiles without the ring (several workgroups per CU), chunks of 4
+// planes or more that give one round of fill_slots workgroups, cached streams (the
+// step; the kernels that write a second grid and never read it again keep
+// nontemporal ones).  Step, FP32 order 8: 128^3 8.4 (was 21), 160^3 16 (27), 200^3
+// 28.5 (39), order 16 37 (56); FP64 150^3 25 (31); FP32 storage with FP64 compute
+// 200^3 31 (41); Laplacian 160^3 12.4 (21), 256^3 order 12 46 (61); D2 of 160^3
+// 8.2-8.5 (12-13).  32 lanes for the kernels that keep twice the registers (FP64
+// values, the step and the Laplacian from order 10 on: 200^3 order 12 34 against
+// 37).  Up to 200 MB; the step but for FP32 to order 8 up to 225 MB (this shape /
+// the one below at 216-221 MB: FP64 order 4-16 49 / 64, 43 / 65, 54 / 68, 49 / 58,
+// FP32 order 12 52 / 84, with FP64 compute order 4 / 8 57 / 67, 50 / 67, FP32 order
+// 4 / 8 64 / 59, 51 / 49; at 290-300 MB it is slower in all but order 16).
 //
 // Larger grids, the fused step:
 //  * FP32 to order 8: 128 x 8 with the ring, fitted to the row, where the row is
 //    wider than one tile of 64 lanes: 300^3 84 (64 x 16: 84), 400^3 190 (195),
 //    600^3 733 (769), 700^3 1064 (1206), 800^3 1763 (1828), 1000^3 2990 (3120);
+//    flat grids can lose (600 x 600 x 40 order 8, 14 %);
 //  * FP32 orders 14 and 16: 32 x 16 without the ring: 450 x 350 x 300 184 / 187
 //    (was 268 / 198);
-//  * FP64 up to 900 MB: 32 x 16 without the ring: 300^3 order 8 164 (177), 320 x
-//    300 x 310 order 4 / 12 166 / 184 (182 / 217); 400^3 and more 64 x 8 with it;
+//  * FP64 orders 6 to 12 up to 900 MB: 32 x 16 without the ring: 300^3 order 8 / 12
+//    164 / 171 (177 / 199), 320^3 order 8 212 (230), 336^3 286 (266); order 4 from
+//    600 MB on only (300^3 164 against 177, 240^3 85 against 80 below); order 2
+//    (240^3 85 against 77) and orders 14 and 16 (2-5 %) are faster without it;
 //  * FP32 storage with FP64 compute: from order 10 32 x 8 without the ring,
-//    nontemporal (400^3 order 12 303, was 406); below, up to 450 MB the same in
-//    12-plane chunks (300^3 100, was 112), up to 2.4 GB 64 x 8 with the ring
-//    (400^3 order 4 / 8 217 / 228, was 234 / 267).
+//    nontemporal (400^3 order 12 303, was 406); below, the same in 12-plane chunks up
+//    to 450 MB (300^3 100, was 112), order 4 up to 900 MB (340^3 121 against 150 with
+//    64 x 8 and the ring, 412^3 231 / 236), order 8 up to 700 MB (336^3 135 / 143,
+//    408^3 274 / 235), then 64 x 8 with the ring (400^3 order 4 / 8 217 / 228, was
+//    234 / 267), orders 2 and 4 up to 2.4 GB (572^3 634, 703 without the ring),
+//    orders 6 and 8 up to 1.4 GB (456^3 362 / 382, 520^3 692 / 591).
 template <typename TS, typename TC, int R, int MODE>
 inline TileCfg default_shape(const hsx_grid *g)
 {
     constexpr bool FP32 = sizeof(TS) == 4 && sizeof(TC) == 4, FP64 = sizeof(TS) == 8;
-    constexpr int VW = 16 / sizeof(TS), GRIDS = mode_ac2(MODE) ? 3 : 2;
-    const int64_t bytes = g->n1 * g->n2 * g->n3 * (int64_t)sizeof(TS) * GRIDS;
+    constexpr int VW = 16 / sizeof(TS);
+    constexpr bool D12 = !Tiled<TS, TC, R, VW, 64, 8, MODE, false>::NEED_Z, D = D12 || MODE == MODE_D2Z || MODE == MODE_D1Z;
+    const int64_t bytes = shape_bytes<TS, MODE>(g);
     const int64_t N1 = g->inner[1] - g->inner[0] + 1;
     TileCfg c = {0, 0, 0, 0};
-    if (bytes <= 200000000) {
-        c.lx = std::min(pick_lx(g, VW, c), FP32 && R <= 4 ? 64 : 32);
+    if (bytes <= (mode_ac2(MODE) && !(FP32 && R <= 4) ? 225000000 : 200000000)) {
+        const bool wide = FP32 ? D || R <= 4 : FP64 ? D12 && R >= 2 && R <= 4 && bytes > 100000000 : D && R <= 4;
+        c.lx = std::min(pick_lx(g, VW, c), wide ? 64 : 32);
         c.by = 8;
         c.flags = HSX_TILE_NO_RING | (mode_ac2(MODE) ? HSX_TILE_CACHED : HSX_TILE_NT) | TILE_FILL;
         return c;
@@ -1154,17 +1205,17 @@ inline TileCfg default_shape(const hsx_grid *g)
             c.flags = HSX_TILE_NO_RING | HSX_TILE_NT;
         }
     } else if (FP64) {
-        if (bytes <= 900000000) {
+        if (R >= 2 && R <= 6 && bytes <= 900000000 && (R > 2 || bytes > 600000000)) {
             c.lx = 32;
             c.by = 16;
             c.flags = HSX_TILE_NO_RING | HSX_TILE_NT;
         }
-    } else if (R >= 5 || bytes <= 450000000) {
+    } else if (R >= 5 || bytes <= (R == 2 ? 900000000 : R == 4 ? 700000000 : 450000000)) {
         c.lx = 32;
         c.by = 8;
         c.chunk = R >= 5 ? 0 : 12;
         c.flags = HSX_TILE_NO_RING | HSX_TILE_NT;
-    } else if (bytes <= 2400000000) {
+    } else if (bytes <= (R <= 2 ? 2400000000 : 1400000000)) {
         c.lx = 64;
         c.by = 8;
     }
@@ -1197,11 +1248,13 @@ inline int run_tiled_shape(const hsx_grid *g, void *out, const void *prn_in, con
                     cfg.flags |= own.flags & TILE_FILL;
                 }
             }
-            int lx = pick_lx(g, VW, cfg, MODE == MODE_LAP);
+            constexpr bool fp32_vals = sizeof(TS) == 4 && sizeof(TC) == 4;
+            constexpr bool across = !Tiled<TS, TC, RR, VW, 64, 8, MODE, false>::NEED_Z;     // D2, D1 along n1 and n2
+            int lx = pick_lx(g, VW, cfg, MODE == MODE_LAP || (mode_ac2(MODE) && fp32_vals) ||
+                                             (across && sizeof(TS) == 4 && RR >= (fp32_vals ? 5 : 3)));
             // the order-8 Laplacian drops the halo ring, whose halo rows still meet
             // in L2 with two streams instead of four (1000^3 1.84 / 1.88 ms, 800^3
             // 1.11 / 1.24, 700^3 0.70 / 0.79, 500^3 0.237 / 0.258, 400^3 0.131 / 0.141)
-            constexpr bool fp32_vals = sizeof(TS) == 4 && sizeof(TC) == 4;
             const bool dflt = cfg.lx == 0 && cfg.by == 0;
             if (fp32_vals && dflt && MODE == MODE_LAP && RR == 2 && wide_by_default(g)) lx = 128;
             if (fp32_vals && dflt && cfg.flags == 0 && MODE == MODE_LAP && RR == 4) cfg.flags = HSX_TILE_NO_RING;

@@ -121,7 +121,8 @@ static TileCfg cached_shape(const hsx_grid *g)
             c = default_shape<TS, TC, R, MODE_AC2>(g);
             const int64_t w = c.lx * (16 / (int64_t)sizeof(TS));
             const int64_t tiles = (g->inner[1] - g->inner[0] + w) / w * ((g->inner[3] - g->inner[2] + c.by) / c.by);
-            c.chunk = (int)chunk_one_round(g->inner[5] - g->inner[4] + 1, R, tiles, 2 * device_cus(), 4);
+            c.chunk = (int)chunk_one_round(g->inner[5] - g->inner[4] + 1, R, tiles,
+                                           fill_slots(c.lx * c.by, fill_threads<TS, R, MODE_AC2>(0)), 4);
             c.flags &= ~TILE_FILL;
             return HSX_OK;
         });

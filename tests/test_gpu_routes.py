@@ -164,3 +164,27 @@ def test_a_partly_given_shape_keeps_the_own_tile(capi, n, order, prec, flags):
     assert flagged == own                      # flags: the own choice of the ring, other streams
     for x in got[1:]:
         _same(x[1], got[0][1])
+
+
+# rows of few lanes, whose workgroups have 72 to 256 threads
+NARROW = [((64, 300, 200), 8, "f32"), ((61, 61, 700), 4, "f32"), ((40, 300, 300), 8, "f32"), ((64, 400, 100), 6, "f32c64"),
+          ((250, 120, 200), 12, "f32c64"), ((200, 190, 180), 12, "f32")]
+
+
+@pytest.mark.parametrize("n,order,prec", NARROW)
+def test_narrow_tiles_fill_the_chip(capi, n, order, prec):
+    """grids in the caches: two workgroups per CU are a full launch only where a
+    workgroup has 400 threads or more; smaller ones come in larger numbers"""
+    p = make_layout(3, n, order)
+    g = capi.hsx_grid(p, compute_fp64=prec == "f32c64")
+    cus = capi.device_info(0)["compute_units"]
+    a, b, c = (capi.DeviceArray(p.npoint * 4) for _ in range(3))
+    for d in (a, b, c):
+        capi.array_op(g, capi.HSX_ARRAY_FILL, d, val=0.0)
+    capi.sync()
+    for op in (lambda s: capi.ac2_step(g, a, b, c, stream=s), lambda s: capi.laplacian(g, b, a, stream=s),
+               lambda s: capi.fd_d2(g, 0, b, a, stream=s), lambda s: capi.fd_d1(g, 1, b, a, stream=s)):
+        ((grid, block, lds),) = launches(capi, op)
+        print(f"n={n} order={order} {prec}: {grid[0]} workgroups of {block[0]}", flush=True)
+        assert block[1] == 1 and block[0] <= 512         # a tile of the cached shape
+        assert block[0] >= 400 or grid[0] > 2 * cus
