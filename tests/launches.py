@@ -14,9 +14,9 @@ class _KernelNodeParams(ctypes.Structure):      # hipKernelNodeParams
                 ("params", ctypes.c_void_p), ("lds", ctypes.c_uint32)]
 
 
-def launches(capi, call):
-    """call(stream) -> [(workgroups, threads, LDS bytes)] of its kernels; it is
-    run once before, for what a first call sets up"""
+def launches(capi, call, func=False):
+    """call(stream) -> [(workgroups, threads, LDS bytes)] of its kernels (func: and
+    their handles); it is run once before, for what a first call sets up"""
     hip = capi.lib()                            # the library's own HIP runtime
     stream, graph, n = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_size_t(0)
 
@@ -37,7 +37,8 @@ def launches(capi, call):
         for node in nodes:
             k = _KernelNodeParams()
             ok(hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(k)))
-            out.append(((k.grid.x, k.grid.y, k.grid.z), (k.block.x, k.block.y, k.block.z), k.lds))
+            out.append(((k.grid.x, k.grid.y, k.grid.z), (k.block.x, k.block.y, k.block.z), k.lds)
+                       + ((k.func,) if func else ()))
         ok(hip.hipGraphDestroy(graph))
         return out
     finally:

@@ -188,3 +188,16 @@ def test_narrow_tiles_fill_the_chip(capi, n, order, prec):
         print(f"n={n} order={order} {prec}: {grid[0]} workgroups of {block[0]}", flush=True)
         assert block[1] == 1 and block[0] <= 512         # a tile of the cached shape
         assert block[0] >= 400 or grid[0] > 2 * cus
+
+
+@pytest.mark.parametrize("fp64", [False, True])
+def test_n1_faces_alone_keep_their_kernel(capi, fp64):
+    """faces along n1 only, rows of whole vectors: the kernel of the row ends, one
+    launch; with other faces the one that leaves their rows out"""
+    p = make_layout(3, (60, 50, 40), 8, fp64=fp64)
+    g = capi.hsx_grid(p)
+    u = _dev(capi, np.zeros(p.npoint, p.dtype))
+    run = {m: launches(capi, lambda s: capi.free_surface(g, u, face_mask=m, stream=s), func=True) for m in (1, 3, 7, 63)}
+    assert all(len(x) == 1 for x in run.values())
+    kernel = {m: x[0][3] for m, x in run.items()}
+    assert kernel[1] == kernel[3] != kernel[7] == kernel[63]
