@@ -1096,7 +1096,7 @@ int bc_batch_fs_launch(int storage, int nshots, void *const *d_fields, const N1F
     const uint32_t nb1 = (uint32_t)std::max<int64_t>(1, std::min<int64_t>((most + 255) / 256, 4096));
     const uint32_t nb2 = (uint32_t)std::max<int64_t>(1, std::min<int64_t>((most_plane + 255) / 256, 4096));
     const dim3 both(nbn + 6 * nb1, (unsigned)nshots);
-    auto launch = [&](auto ts) {
+    auto launch = [&](auto ts) -> int {
         using TS = decltype(ts);
         TS *const *u = (TS *const *)d_fields;
         switch (nh) {
@@ -1108,12 +1108,9 @@ int bc_batch_fs_launch(int storage, int nshots, void *const *d_fields, const N1F
         HSX_LAUNCHED("k_bc_n1_mirror_batch");
         hipLaunchKernelGGL(k_bc_zero_batch<TS>, dim3(nb2, 6 * nshots), dim3(256), 0, s, u, d_sets);
         HSX_LAUNCHED("k_bc_zero_batch");
+        return HSX_OK;
     };
-    if (storage == HSX_FP64)
-        launch(0.0);
-    else
-        launch(0.0f);
-    return HSX_OK;
+    return storage == HSX_FP64 ? launch(0.0) : launch(0.0f);
 }
 
 // ---- leapfrog update of the split propagator (src/grid.cpp:4579-4610) -----------
